@@ -95,6 +95,26 @@ int tvllm_apply_table_updates(int64_t* table, int64_t table_size,
                               const int64_t* updates, int64_t capacity,
                               tvllm_stream_t stream);
 
+/* tvllm_apply_table_updates and tvllm_resolve_tokens (below) in one launch:
+ * the head of a decode step. The buffers of the two must not overlap. */
+int tvllm_begin_decode(int64_t* table, int64_t table_size, const int64_t* updates,
+                       int64_t capacity, int64_t* tokens, const int64_t* src,
+                       const int64_t* prev, int64_t n, int64_t prev_count,
+                       tvllm_stream_t stream);
+
+/* out[t] = embed[ids[t]], cos_out[t] = cos[positions[t]], sin_out[t] =
+ * sin[positions[t]]: the embedding and RoPE rows of a step's tokens, bit
+ * copies in one launch. embed [vocab, width], cos and sin [max_position,
+ * half], outputs [tokens, width] and [tokens, half], all dense and 16-byte
+ * aligned, width and half multiples of 8. An id or position outside its
+ * table gives a row of NaNs and reads nothing.
+ * Replaces: nn.Embedding and RotaryEmbedding's gathers (reference
+ *           tinyvllm/models/qwen3.py, layers.py:167-245). */
+int tvllm_embed_rope(const int64_t* ids, const int64_t* positions, int64_t tokens,
+                     const void* embed, int64_t vocab, int64_t width, const void* cos,
+                     const void* sin, int64_t max_position, int64_t half, void* out,
+                     void* cos_out, void* sin_out, int dtype, tvllm_stream_t stream);
+
 /* Bytes of device workspace tvllm_paged_decode needs for this geometry
  * (split-K partial results). 0 means no workspace is needed.
  * max_context_len bounds the context of any row (the engine's

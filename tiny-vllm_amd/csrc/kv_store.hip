@@ -203,15 +203,46 @@ extern "C" int tvllm_store_kv(const void* key, const void* value,
 namespace tvllm {
 namespace {
 
-__global__ void __launch_bounds__(256)
-apply_table_updates_kernel(int64_t* __restrict__ table, int64_t table_size,
-                           const int64_t* __restrict__ updates, int64_t capacity) {
+__device__ __forceinline__ void apply_updates(int64_t* __restrict__ table, int64_t table_size,
+                                              const int64_t* __restrict__ updates,
+                                              int64_t capacity, int block, int blocks) {
     const int64_t n = min(updates[0], capacity);
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x) {
+    for (int64_t i = int64_t(block) * blockDim.x + threadIdx.x; i < n;
+         i += int64_t(blocks) * blockDim.x) {
         const int64_t index = updates[1 + 2 * i];
         if (index >= 0 && index < table_size) table[index] = updates[2 + 2 * i];
     }
+}
+
+__global__ void __launch_bounds__(256)
+apply_table_updates_kernel(int64_t* __restrict__ table, int64_t table_size,
+                           const int64_t* __restrict__ updates, int64_t capacity) {
+    apply_updates(table, table_size, updates, capacity, blockIdx.x, gridDim.x);
+}
+
+// Both heads of a decode step in one launch (they touch different buffers):
+// the first `table_blocks` workgroups apply the table updates, the others
+// take each row's token from the previous step's samples where its source
+// says so. Two launches of ~3 us each otherwise.
+__global__ void __launch_bounds__(256)
+begin_decode_kernel(int64_t* __restrict__ table, int64_t table_size,
+                    const int64_t* __restrict__ updates, int64_t capacity, int table_blocks,
+                    int64_t* __restrict__ tokens, const int64_t* __restrict__ src,
+                    const int64_t* __restrict__ prev, int64_t n, int64_t prev_count) {
+    if (int(blockIdx.x) < table_blocks) {
+        apply_updates(table, table_size, updates, capacity, blockIdx.x, table_blocks);
+        return;
+    }
+    const int64_t i = int64_t(blockIdx.x - table_blocks) * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int64_t s = src[i];
+    if (s >= 0 && s < prev_count) tokens[i] = prev[s];
+}
+
+// Enough threads for a typical step (a page per row); larger uploads (rows
+// entering decode with whole tables) loop.
+int update_blocks(int64_t capacity) {
+    return int(std::min<int64_t>((capacity + 255) / 256, 64));
 }
 
 }  // namespace
@@ -225,10 +256,25 @@ extern "C" int tvllm_apply_table_updates(int64_t* table, int64_t table_size,
                 "apply_table_updates: negative sizes");
     if (capacity == 0) return TVLLM_OK;
     TVLLM_CHECK(table && updates, "apply_table_updates: null pointer");
-    // Enough threads for a typical step (a page per row); larger uploads
-    // (rows entering decode with whole tables) loop.
-    const int blocks = int(std::min<int64_t>((capacity + 255) / 256, 64));
-    apply_table_updates_kernel<<<blocks, 256, 0, as_hip(stream)>>>(table, table_size,
-                                                                     updates, capacity);
+    apply_table_updates_kernel<<<update_blocks(capacity), 256, 0, as_hip(stream)>>>(
+        table, table_size, updates, capacity);
     return launch_status("apply_table_updates");
+}
+
+extern "C" int tvllm_begin_decode(int64_t* table, int64_t table_size, const int64_t* updates,
+                                  int64_t capacity, int64_t* tokens, const int64_t* src,
+                                  const int64_t* prev, int64_t n, int64_t prev_count,
+                                  tvllm_stream_t stream) {
+    using namespace tvllm;
+    TVLLM_CHECK(table_size >= 0 && capacity >= 0 && n >= 0 && prev_count >= 0,
+                "begin_decode: negative sizes");
+    TVLLM_CHECK(n <= int64_t(INT32_MAX) / 2, "begin_decode: too many tokens");
+    if (capacity == 0 && n == 0) return TVLLM_OK;
+    TVLLM_CHECK(capacity == 0 || (table && updates), "begin_decode: null table");
+    TVLLM_CHECK(n == 0 || (tokens && src && (prev || prev_count == 0)),
+                "begin_decode: null tokens");
+    const int table_blocks = capacity ? update_blocks(capacity) : 0;
+    begin_decode_kernel<<<table_blocks + int((n + 255) / 256), 256, 0, as_hip(stream)>>>(
+        table, table_size, updates, capacity, table_blocks, tokens, src, prev, n, prev_count);
+    return launch_status("begin_decode");
 }

@@ -68,6 +68,9 @@ _SIGNATURES: dict[str, tuple[type, list[type]]] = {
                             _I64, _INT, _P]),
     "tvllm_resolve_tokens": (_INT, [_P, _P, _P, _I64, _I64, _P]),
     "tvllm_apply_table_updates": (_INT, [_P, _I64, _P, _I64, _P]),
+    "tvllm_begin_decode": (_INT, [_P, _I64, _P, _I64, _P, _P, _P, _I64, _I64, _P]),
+    "tvllm_embed_rope": (_INT, [_P, _P, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _P, _P, _P,
+                                _INT, _P]),
     "tvllm_paged_prefill": (_INT, [_P, _I64, _I64, _P, _P, _P, _I64, _I64, _P,
                                    _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                    _I64, _I64, _I64, _I64, _F32, _P, _I64, _INT, _INT, _F32,

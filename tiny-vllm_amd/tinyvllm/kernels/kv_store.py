@@ -65,3 +65,22 @@ def apply_table_updates(table: torch.Tensor, updates: torch.Tensor) -> None:
     capacity = (updates.numel() - 1) // 2
     check(lib.tvllm_apply_table_updates(table.data_ptr(), table.numel(), updates.data_ptr(),
                                         capacity, stream_of(device)))
+
+
+def begin_decode(table: torch.Tensor, updates: torch.Tensor, tokens: torch.Tensor,
+                 src: torch.Tensor, prev: torch.Tensor) -> None:
+    """``apply_table_updates(table, updates)`` and ``resolve_tokens(tokens,
+    src, prev)`` in one launch: the head of a decode step."""
+    lib = load_kernels()
+    device = require_gpu(table, updates, tokens, src, prev)
+    for tensor in (table, updates, tokens, src, prev):
+        if tensor.dtype != torch.long or tensor.dim() != 1 or not tensor.is_contiguous():
+            raise RuntimeError("begin_decode takes contiguous 1-D int64 tensors")
+    if updates.numel() < 1:
+        raise RuntimeError("updates needs its count word")
+    if src.shape != tokens.shape:
+        raise RuntimeError("src must have one entry per token")
+    check(lib.tvllm_begin_decode(
+        table.data_ptr(), table.numel(), updates.data_ptr(), (updates.numel() - 1) // 2,
+        tokens.data_ptr(), src.data_ptr(), prev.data_ptr(), tokens.numel(), prev.numel(),
+        stream_of(device)))

@@ -240,3 +240,38 @@ def qk_norm_rope_store(
             float(k_scale), float(v_scale), stream_of(device),
         ))
     return q_out, k_out
+
+
+def embed_rope(
+    input_ids: torch.Tensor,
+    positions: torch.Tensor,
+    embedding: torch.Tensor,
+    cos: torch.Tensor,
+    sin: torch.Tensor,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """A step's embedding rows [tokens, width] and its cos / sin rows [tokens,
+    1, half] in one launch: bit copies of ``embedding[input_ids]``,
+    ``cos[positions]`` and ``sin[positions]`` (tables ``[rows, columns]`` of
+    one half dtype, columns a multiple of 8). Ids and positions must lie in
+    their tables; others give rows of NaNs."""
+    lib = load_kernels()
+    device = require_gpu(input_ids, positions, embedding, cos, sin)
+    for tensor in (input_ids, positions):
+        if tensor.dtype != torch.long or tensor.dim() != 1 or not tensor.is_contiguous():
+            raise RuntimeError("ids and positions must be contiguous 1-D int64 tensors")
+    if positions.shape != input_ids.shape or cos.shape != sin.shape:
+        raise RuntimeError("ids and positions, cos and sin must align")
+    for table in (embedding, cos, sin):
+        if table.dim() != 2 or not table.is_contiguous() or table.dtype != embedding.dtype:
+            raise RuntimeError("tables must be contiguous 2-D tensors of one dtype")
+    tokens = input_ids.numel()
+    (vocab, width), (rows, half) = embedding.shape, cos.shape
+    out = torch.empty((tokens, width), dtype=embedding.dtype, device=device)
+    cos_out = torch.empty((tokens, 1, half), dtype=embedding.dtype, device=device)
+    sin_out = torch.empty((tokens, 1, half), dtype=embedding.dtype, device=device)
+    check(lib.tvllm_embed_rope(
+        input_ids.data_ptr(), positions.data_ptr(), tokens, embedding.data_ptr(), vocab, width,
+        cos.data_ptr(), sin.data_ptr(), rows, half, out.data_ptr(), cos_out.data_ptr(),
+        sin_out.data_ptr(), dtype_code(embedding.dtype), stream_of(device),
+    ))
+    return out, cos_out, sin_out

@@ -244,15 +244,20 @@ class RotaryEmbedding(nn.Module):
         self, positions: torch.Tensor, dtype: torch.dtype,
     ) -> tuple[torch.Tensor, torch.Tensor]:
         """cos, sin of ``positions`` as [tokens, 1, head_dim / 2] in ``dtype``."""
+        tables = self.tables(dtype)
+        cos = tables[0].index_select(0, positions).unsqueeze(1)
+        sin = tables[1].index_select(0, positions).unsqueeze(1)
+        return cos, sin
+
+    def tables(self, dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+        """The cos and sin tables [max_position, head_dim / 2] in ``dtype``."""
         tables = self._cast.get(dtype)
         if tables is None:
             if self.cos.is_cuda and torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("RoPE tables must be cast before graph capture")
             tables = (self.cos.to(dtype), self.sin.to(dtype))
             self._cast[dtype] = tables
-        cos = tables[0].index_select(0, positions).unsqueeze(1)
-        sin = tables[1].index_select(0, positions).unsqueeze(1)
-        return cos, sin
+        return tables
 
 
 class SiluAndMul(nn.Module):

@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from tinyvllm._validation import _check_positive_int
-from tinyvllm.kernels.pointwise import qk_norm_rope
+from tinyvllm.kernels.pointwise import embed_rope, qk_norm_rope
 from tinyvllm.layers import (
     PackedLinear, RMSNorm, RotaryEmbedding, SiluAndMul, SplitKLinear, SplitKPartials,
 )
@@ -231,6 +231,26 @@ class Qwen3Model(nn.Module):
         self.norm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps,
                             device=device, dtype=dtype)
 
+    def _embed(self, input_ids: torch.Tensor, positions: torch.Tensor):
+        """Embedding rows and (cos, sin) rows of the step's tokens: one launch
+        for half-precision tables on the GPU with rows of whole 16-byte units
+        (outside autograd and without hooks, which only the modules' own
+        calls serve), the modules otherwise."""
+        weight = self.embed_tokens.weight
+        if (weight.is_cuda and input_ids.is_cuda and not torch.is_grad_enabled()
+                and weight.dtype in (torch.float16, torch.bfloat16)
+                and self.config.hidden_size % 8 == 0 and self.config.head_dim % 16 == 0
+                and weight.is_contiguous() and input_ids.is_contiguous()
+                and positions.is_contiguous()
+                and not (self.embed_tokens._forward_hooks or self.embed_tokens._forward_pre_hooks
+                         or self.rotary_emb._forward_hooks
+                         or self.rotary_emb._forward_pre_hooks)):
+            hidden, cos, sin = embed_rope(input_ids, positions, weight,
+                                          *self.rotary_emb.tables(weight.dtype))
+            return hidden, (cos, sin)
+        hidden = self.embed_tokens(input_ids)
+        return hidden, self.rotary_emb(positions, hidden.dtype)
+
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, *,
                 attention: AttentionBackend) -> torch.Tensor:
         if input_ids.ndim != 1 or input_ids.numel() == 0:
@@ -239,8 +259,7 @@ class Qwen3Model(nn.Module):
             raise TypeError("input_ids and positions must use torch.long")
         if positions.shape != input_ids.shape or positions.device != input_ids.device:
             raise ValueError("positions must align with input_ids on the same device")
-        hidden = self.embed_tokens(input_ids)
-        rope = self.rotary_emb(positions, hidden.dtype)
+        hidden, rope = self._embed(input_ids, positions)
         residual = None
         for index, layer in enumerate(self.layers):
             hidden, residual = layer(hidden, rope, residual=residual, layer_idx=index,

@@ -15,8 +15,9 @@ from __future__ import annotations
 
 import torch
 
+from tinyvllm.kernels.kv_store import begin_decode
 from tinyvllm.kernels.paged_decode import decode_split_plan
-from tinyvllm.kernels.sampling import resolve_tokens, sample
+from tinyvllm.kernels.sampling import sample
 from tinyvllm.paged_kv import PagedKVCache
 from tinyvllm.runtime.attention import HipAttention
 from tinyvllm.runtime.inputs import DecodeInputs
@@ -122,8 +123,8 @@ class DecodeGraphs:
         sources = inputs.d["sources"][:size]
 
         def step():
-            inputs.apply_table_updates()
-            resolve_tokens(model_input.input_ids, sources, self.tokens)
+            begin_decode(inputs.table, inputs.d["updates"], model_input.input_ids, sources,
+                         self.tokens)
             attention = HipAttention(model_input, cache, decode_workspace=workspace)
             hidden = model(model_input.input_ids, model_input.positions, attention=attention)
             logits = model.compute_logits(hidden)
