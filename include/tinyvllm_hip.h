@@ -338,13 +338,16 @@ int tvllm_argmax(const void* logits, int64_t rows, int64_t vocab,
  *   out[r] = argmax_{kept i} p_i / E_i,  E_i ~ Exp(1) from a counter-based
  *   Philox4x32-10 stream keyed by (seeds[r], counters[r], i).
  * temperature > 0 samples; temperature 0 rows take the argmax.
- * workspace (optional, 16-byte aligned): tvllm_sample_workspace_size(rows,
- * vocab) bytes of per-span argmax partials, so that each row's scan is
- * spread over several workgroups (an extra launch); with workspace_bytes 0
- * each row's workgroup scans the row alone. Same result either way.
+ * workspace (optional, 16-byte aligned): with
+ * tvllm_sample_split_workspace_size(rows, vocab) bytes every pass over a row
+ * is spread over several workgroups (four launches); with
+ * tvllm_sample_workspace_size(rows, vocab) bytes only the search for the
+ * row's maximum is (two launches); with workspace_bytes 0 each row's
+ * workgroup draws alone. Same result in all three.
  * Replaces: TorchSampler._sample_batch (reference tinyvllm/sampling.py:75-164);
  *           the noise stream differs from torch.Generator's. */
 int64_t tvllm_sample_workspace_size(int64_t rows, int64_t vocab);
+int64_t tvllm_sample_split_workspace_size(int64_t rows, int64_t vocab);
 int tvllm_sample(const void* logits, int64_t rows, int64_t vocab,
                  int64_t row_stride, const float* temperature,
                  const int64_t* top_k, const float* top_p,

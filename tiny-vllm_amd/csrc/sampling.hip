@@ -61,21 +61,6 @@ __device__ void block_argmax_w(float& v, int64_t& idx) {
     __syncthreads();
 }
 
-// Block-wide argmax; every thread gets the result.
-__device__ void block_argmax(float& v, int64_t& idx) {
-    __shared__ float sv[kWaves];
-    __shared__ int64_t si[kWaves];
-    wave_argmax(v, idx);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { sv[w] = v; si[w] = idx; }
-    __syncthreads();
-    v = sv[0];
-    idx = si[0];
-    for (int i = 1; i < kWaves; ++i)
-        if (better(sv[i], si[i], v, idx)) { v = sv[i]; idx = si[i]; }
-    __syncthreads();
-}
-
 template <typename T, bool VEC>
 __global__ void __launch_bounds__(kThreads)
 argmax_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
@@ -135,7 +120,7 @@ __device__ __forceinline__ bool kept(const Cut& c, uint32_t key, int64_t i) {
 // Finds the first element, in (key descending, index ascending) order among
 // elements with in(i), whose inclusive cumulative weight exceeds `target`.
 // weight(i) is 1 (MASS = false) or the fixed-point probability mass.
-template <typename T, bool MASS, typename In>
+template <typename T, bool MASS, int NT, typename In>
 __device__ Cut radix_cut(const T* row, int64_t vocab, const RowCtx& ctx,
                          uint64_t target, In&& in) {
     __shared__ uint64_t hist[256];
@@ -145,9 +130,9 @@ __device__ Cut radix_cut(const T* row, int64_t vocab, const RowCtx& ctx,
     uint32_t prefix = 0;
     uint64_t above = 0;
     for (int shift = 24; shift >= 0; shift -= 8) {
-        for (int b = threadIdx.x; b < 256; b += kThreads) hist[b] = 0;
+        for (int b = threadIdx.x; b < 256; b += NT) hist[b] = 0;
         __syncthreads();
-        for (int64_t i = threadIdx.x; i < vocab; i += kThreads) {
+        for (int64_t i = threadIdx.x; i < vocab; i += NT) {
             if (!in(i)) continue;
             const float s = score_of(row, i, ctx);
             const uint32_t k = fkey(s);
@@ -186,7 +171,7 @@ __device__ Cut radix_cut(const T* row, int64_t vocab, const RowCtx& ctx,
         __shared__ uint64_t s_w;
         if (threadIdx.x == 0) s_w = 0;
         __syncthreads();
-        for (int64_t i = threadIdx.x; i < vocab; i += kThreads) {
+        for (int64_t i = threadIdx.x; i < vocab; i += NT) {
             if (!in(i)) continue;
             const float s = score_of(row, i, ctx);
             if (fkey(s) == prefix) { s_w = mass_of(s); break; }
@@ -203,9 +188,9 @@ __device__ Cut radix_cut(const T* row, int64_t vocab, const RowCtx& ctx,
     uint32_t iprefix = 0;
     uint64_t below = 0;
     for (int shift = 16; shift >= 0; shift -= 8) {
-        for (int b = threadIdx.x; b < 256; b += kThreads) ihist[b] = 0;
+        for (int b = threadIdx.x; b < 256; b += NT) ihist[b] = 0;
         __syncthreads();
-        for (int64_t i = threadIdx.x; i < vocab; i += kThreads) {
+        for (int64_t i = threadIdx.x; i < vocab; i += NT) {
             if (!in(i)) continue;
             const uint32_t ui = static_cast<uint32_t>(i);
             if (shift < 16 && ((ui ^ iprefix) >> (shift + 8)) != 0) continue;
@@ -348,12 +333,41 @@ struct ArgPart {
     int32_t i;  // -1: empty span
 };
 
+// Bins of width 1/64 over s in (-32, 0]. Monotonic in s (a product with a
+// power of two, truncated), so bins respect the key order. The last bin takes
+// everything below: its masses are 0 in 2^-40 fixed point (e^-31.9 = 1.4e-14),
+// and it is not counted. 16-bit logits of a trained or random head put tens
+// to a few hundred tokens in a bin; 4096 list entries hold bins of heads with
+// a standard deviation down to about 0.25.
+constexpr int kBins = 2048;
+constexpr float kBinScale = 64.f;
+constexpr int kListCap = 4096;
+
+__device__ __forceinline__ int bin_of(float s) {
+    return int(fminf(-s * kBinScale, float(kBins - 1)));
+}
+
+struct alignas(16) RowState {
+    unsigned long long bins[kBins];
+    unsigned long long list[kListCap];  // key << 32 | ~index
+    unsigned long long rest;            // weight that the list's kept part must exceed
+    uint32_t listed;                    // tokens offered to the list
+    uint32_t whole;                     // the row is drawn by one workgroup
+};
+
 template <typename T, bool VEC>
 __global__ void __launch_bounds__(kPartThreads)
 argmax_part_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride, int nparts,
-                   ArgPart* __restrict__ parts) {
+                   const float* __restrict__ temperature, ArgPart* __restrict__ parts,
+                   RowState* __restrict__ states) {
     const int r = blockIdx.x / nparts;
     const int span = blockIdx.x - r * nparts;
+    // The spans share the clearing of a sampled row's state.
+    if (states != nullptr && temperature[r] > 0.f) {
+        for (int b = span * kPartThreads + threadIdx.x; b < kBins; b += nparts * kPartThreads)
+            states[r].bins[b] = 0;
+        if (span == 0 && threadIdx.x == 0) states[r].listed = 0;
+    }
     const T* row = logits + int64_t(r) * stride;
     const int64_t begin = int64_t(span) * kPartSpan;
     const int64_t end = min(vocab, begin + kPartSpan);
@@ -409,6 +423,82 @@ argmax_part_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride, 
         parts[blockIdx.x] = ArgPart{best, bi == INT64_MAX ? -1 : int32_t(bi)};
 }
 
+// One element's race value s - log(E), E ~ Exp(1) from word i % 4 of the
+// Philox block i / 4 of the row's (seed, counter) stream.
+__device__ __forceinline__ float race_value(float s, uint32_t bits) {
+    const float u = (float(bits >> 8) + 0.5f) * (1.0f / 16777216.0f);
+    const float e = -logf(u);
+    return s - logf(e);
+}
+
+struct Noise {
+    uint2 key;
+    uint64_t step;
+    __device__ __forceinline__ uint4 block(int64_t i) const {
+        return philox4x32_10(
+            make_uint4(static_cast<uint32_t>(i >> 2), static_cast<uint32_t>(i >> 34),
+                       static_cast<uint32_t>(step), static_cast<uint32_t>(step >> 32)),
+            key);
+    }
+    __device__ __forceinline__ uint32_t bits(int64_t i) const {
+        const uint4 r = block(i);
+        const int w = int(i & 3);
+        return w == 0 ? r.x : w == 1 ? r.y : w == 2 ? r.z : r.w;
+    }
+};
+
+__device__ __forceinline__ Noise noise_of(int64_t seed, int64_t counter) {
+    return Noise{make_uint2(static_cast<uint32_t>(seed),
+                            static_cast<uint32_t>(uint64_t(seed) >> 32)),
+                 static_cast<uint64_t>(counter)};
+}
+
+// One row's draw by one workgroup of NT threads, whatever the row holds
+// (radix selection over the whole row): rows without a workspace, and those
+// whose boundary bin holds more tokens than the gathered list.
+template <typename T, int NT>
+__device__ int64_t sample_row(const T* row, int64_t vocab, const RowCtx& ctx, int64_t k, float p,
+                              const Noise& noise) {
+    Cut kcut{0u, 0, true};
+    if (k > 0 && k < vocab) {
+        kcut = radix_cut<T, false, NT>(row, vocab, ctx, uint64_t(k - 1),
+                                       [](int64_t) { return true; });
+    }
+    auto in_k = [&](int64_t i) {
+        return kcut.all || kept(kcut, fkey(score_of(row, i, ctx)), i);
+    };
+
+    Cut pcut{0u, 0, true};
+    if (p < 1.f) {
+        // Z = total mass of the top-k candidates (the softmax denominator).
+        __shared__ unsigned long long s_z;
+        if (threadIdx.x == 0) s_z = 0;
+        __syncthreads();
+        unsigned long long z = 0;
+        for (int64_t i = threadIdx.x; i < vocab; i += NT)
+            if (in_k(i)) z += mass_of(score_of(row, i, ctx));
+        atomicAdd(&s_z, z);
+        __syncthreads();
+        const uint64_t target = static_cast<uint64_t>(static_cast<double>(p) *
+                                                      static_cast<double>(s_z));
+        pcut = radix_cut<T, true, NT>(row, vocab, ctx, target, in_k);
+    }
+
+    // Exponential race over the kept set: argmax s_i - log(E_i).
+    float bv = -INFINITY;
+    int64_t bidx = INT64_MAX;
+    for (int64_t i = threadIdx.x; i < vocab; i += NT) {
+        const float s = score_of(row, i, ctx);
+        const uint32_t kk = fkey(s);
+        if (!kcut.all && !kept(kcut, kk, i)) continue;
+        if (!pcut.all && !kept(pcut, kk, i)) continue;
+        const float g = race_value(s, noise.bits(i));
+        if (better(g, i, bv, bidx)) { bv = g; bidx = i; }
+    }
+    block_argmax_w<NT / 64>(bv, bidx);
+    return bidx;
+}
+
 template <typename T, bool VEC>
 __global__ void __launch_bounds__(kThreads)
 sample_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
@@ -432,66 +522,366 @@ sample_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
     } else {
         thread_argmax<T, VEC>(row, vocab, best, bi);
     }
-    block_argmax(best, bi);
+    block_argmax_w<kWaves>(best, bi);
     const float temp = temperature[r];
-    if (!(temp > 0.f)) {
-        if (threadIdx.x == 0) out[r] = bi;
-        return;
+    if (temp > 0.f)
+        bi = sample_row<T, kThreads>(row, vocab, RowCtx{best, temp}, top_k[r], top_p[r],
+                                     noise_of(seeds[r], counters[r]));
+    if (threadIdx.x == 0) out[r] = bi;
+}
+
+// ------------------------------------------- sampling split over spans ----
+// With a workspace, a row's passes are spread over its spans (kPartSpan
+// elements each, one 256-thread workgroup): three launches of rows x spans
+// workgroups that each read the row once, and a short one per row, where the
+// one-workgroup kernel reads the row about fifteen times from one CU. 64 rows
+// x 151936 bf16 with mixed filters: 1965 -> 68 us (race about 30, bins 17,
+// finish 10-16, maxima 10: bound by their exponentials, logarithms and Philox
+// blocks and by four launches; 19 MB is 3 us of memory). A batch of greedy
+// rows pays 2 us for the two launches that find nothing to do.
+//
+//   argmax_part_kernel  each span's maximum; clears the row's bins.
+//   bins_kernel         the row maximum from the spans (greedy rows are done);
+//                       adds the span's tokens to the row's bins of s: their
+//                       number (rows with a top-k) or their mass (top-p only).
+//   race_kernel         finds the bin that holds the cut. Tokens in better
+//                       bins are kept whatever happens inside that bin: with
+//                       top-p only they race right here; the cut's own bin
+//                       (with top-k: every bin up to it) is gathered into the
+//                       row's list.
+//   finish_kernel       sorts the list, cuts it exactly, races what is kept
+//                       of it against the spans' winners.
+//
+// The finish is a launch of its own: with the row's last workgroup to finish
+// doing it, the device-wide fence in front of each arrival (1216 of them)
+// cost more than everything else (64 sampled rows: 64-120 us of fences).
+//
+// The sums are integers, so neither the order of the workgroups nor that of
+// the list changes the result: it is the one-workgroup kernel's.
+
+__device__ __forceinline__ ArgPart row_max(const ArgPart* __restrict__ parts, int nparts) {
+    float best = -INFINITY;
+    int64_t bi = INT64_MAX;
+    for (int i = threadIdx.x & 63; i < nparts; i += 64) {
+        const ArgPart p = parts[i];
+        const int64_t pi = p.i < 0 ? INT64_MAX : int64_t(p.i);
+        if (better(p.v, pi, best, bi)) { best = p.v; bi = pi; }
     }
-    const RowCtx ctx{best, temp};
+    wave_argmax(best, bi);  // every wave on its own
+    return ArgPart{best, bi == INT64_MAX ? -1 : int32_t(bi)};
+}
+
+// What a row needs: its list and bins hold counts (top-k) or masses (top-p
+// only); a row that keeps everything needs neither. A row whose maximum is
+// not finite (NaN, infinities) goes to the one-workgroup draw.
+enum class Draw { kGreedy, kAll, kTopK, kTopP, kWhole };
+
+__device__ __forceinline__ Draw draw_of(float temp, float mx, int64_t k, float p, int64_t vocab) {
+    if (!(temp > 0.f)) return Draw::kGreedy;
+    if (!(fabsf(mx) < INFINITY)) return Draw::kWhole;
+    if (k > 0 && k < vocab) return Draw::kTopK;
+    return p < 1.f ? Draw::kTopP : Draw::kAll;
+}
+
+// f(i, logit) for every element of the thread's share of span [begin, end),
+// aligned groups of 8 consecutive elements per vector load when VEC (`end` is
+// a multiple of 8 except in a row's last span).
+template <typename T, bool VEC, typename F>
+__device__ __forceinline__ void for_span(const T* row, int64_t begin, int64_t end, F&& f) {
+    int64_t tail = begin;
+    if constexpr (VEC) {
+        const U16x8* rv = reinterpret_cast<const U16x8*>(row);
+        const uint32_t v0 = uint32_t(begin / 8), v1 = uint32_t(end / 8);
+        if (v0 < v1) {
+        U16x8 raw[kPartVecs];
+#pragma unroll
+        for (int u = 0; u < kPartVecs; ++u) {
+            const uint32_t c = v0 + threadIdx.x + uint32_t(u) * kPartThreads;
+            raw[u] = rv[c < v1 ? c : v0];
+        }
+#pragma unroll
+        for (int u = 0; u < kPartVecs; ++u) {
+            const uint32_t c = v0 + threadIdx.x + uint32_t(u) * kPartThreads;
+            if (c >= v1) break;
+            float x[8];
+            unpack8<T>(raw[u], x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f(int64_t(c) * 8 + e, x[e]);
+        }
+        }
+        tail = int64_t(v1) * 8;
+    }
+    for (int64_t i = tail + threadIdx.x; i < end; i += kPartThreads) f(i, load_logit(row, i));
+}
+
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(kPartThreads)
+bins_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
+            const float* __restrict__ temperature, const int64_t* __restrict__ top_k,
+            const float* __restrict__ top_p, int64_t* __restrict__ out,
+            const ArgPart* __restrict__ parts, int nparts, RowState* __restrict__ states) {
+    __shared__ unsigned long long bins[kBins];
+    const int r = blockIdx.x / nparts;
+    const int span = blockIdx.x - r * nparts;
+    const float temp = temperature[r];
+    if (!(temp > 0.f) && span != 0) return;
+    const ArgPart top = row_max(parts + int64_t(r) * nparts, nparts);
+    const Draw draw = draw_of(temp, top.v, top_k[r], top_p[r], vocab);
+    if (draw == Draw::kGreedy && threadIdx.x == 0) out[r] = top.i;
+    if (draw != Draw::kTopK && draw != Draw::kTopP) return;
+    for (int b = threadIdx.x; b < kBins; b += kPartThreads) bins[b] = 0;
+    __syncthreads();
+    const bool mass = draw == Draw::kTopP;
+    const int64_t begin = int64_t(span) * kPartSpan;
+    for_span<T, VEC>(logits + int64_t(r) * stride, begin, min(vocab, begin + kPartSpan),
+                     [&](int64_t, float x) {
+        const float s = (x - top.v) / temp;
+        const int b = bin_of(s);
+        if (b < kBins - 1) {
+            const unsigned long long w = mass ? mass_of(s) : 1ull;
+            if (w != 0) atomicAdd(&bins[b], w);
+        }
+    });
+    __syncthreads();
+    unsigned long long* const sum = states[r].bins;
+    for (int b = threadIdx.x; b < kBins; b += kPartThreads)
+        if (bins[b] != 0) atomicAdd(&sum[b], bins[b]);
+}
+
+// Exclusive prefix sum over the NT threads of the workgroup; `total` for all.
+template <int NT>
+__device__ uint64_t block_scan(uint64_t v, uint64_t& total) {
+    __shared__ uint64_t wave_total[NT / 64];
+    uint64_t incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t o = __shfl_up(incl, off, 64);
+        if (int(threadIdx.x & 63) >= off) incl += o;
+    }
+    if ((threadIdx.x & 63) == 63) wave_total[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    uint64_t before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        if (w < int(threadIdx.x >> 6)) before += wave_total[w];
+        total += wave_total[w];
+    }
+    __syncthreads();
+    return before + incl - v;
+}
+
+// First position (of n, thread t owning the run [t * per, (t + 1) * per))
+// whose inclusive sum of weight(i) exceeds target: that position and the sum
+// before it, or n and the whole sum where none does.
+template <int NT, typename W>
+__device__ uint64_t first_over(int n, int per, uint64_t target, int& pos, W&& weight) {
+    __shared__ int s_pos;
+    __shared__ uint64_t s_above;
+    const int i0 = min(n, int(threadIdx.x) * per), i1 = min(n, i0 + per);
+    uint64_t mine = 0, total;
+    for (int i = i0; i < i1; ++i) mine += weight(i);
+    uint64_t cum = block_scan<NT>(mine, total);
+    if (threadIdx.x == 0) { s_pos = n; s_above = total; }
+    __syncthreads();
+    if (cum <= target && cum + mine > target) {  // at most one thread
+        int i = i0;
+        for (; i < i1; ++i) {
+            const uint64_t w = weight(i);
+            if (cum + w > target) break;
+            cum += w;
+        }
+        s_pos = i;
+        s_above = cum;
+    }
+    __syncthreads();
+    pos = s_pos;
+    const uint64_t above = s_above;
+    __syncthreads();
+    return above;
+}
+
+__device__ __forceinline__ float key_value(uint32_t key) {  // inverse of fkey
+    return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
+}
+
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(kPartThreads)
+race_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
+            const float* __restrict__ temperature, const int64_t* __restrict__ top_k,
+            const float* __restrict__ top_p, const int64_t* __restrict__ seeds,
+            const int64_t* __restrict__ counters, const ArgPart* __restrict__ parts, int nparts,
+            RowState* __restrict__ states, ArgPart* __restrict__ races) {
+    __shared__ unsigned long long listed[kListCap];  // the span's share of the row's list
+    __shared__ uint32_t s_listed, s_at;
+    const int r = blockIdx.x / nparts;
+    const int span = blockIdx.x - r * nparts;
+    const float temp = temperature[r];
+    if (!(temp > 0.f)) return;  // greedy: answered by bins_kernel
+    if (threadIdx.x == 0) s_listed = 0;
+    __syncthreads();
+    const T* row = logits + int64_t(r) * stride;
     const int64_t k = top_k[r];
     const float p = top_p[r];
+    const Noise noise = noise_of(seeds[r], counters[r]);
+    const RowCtx ctx{row_max(parts + int64_t(r) * nparts, nparts).v, temp};
+    const Draw draw = draw_of(temp, ctx.mx, k, p, vocab);
+    RowState& state = states[r];
 
-    Cut kcut{0u, 0, true};
-    if (k > 0 && k < vocab) {
-        kcut = radix_cut<T, false>(row, vocab, ctx, uint64_t(k - 1),
-                                   [](int64_t) { return true; });
+    int cut = kBins;  // tokens of the bins below it are kept
+    bool whole = draw == Draw::kWhole;
+    uint64_t rest = 0;
+    if (draw == Draw::kTopK || draw == Draw::kTopP) {
+        constexpr int kPer = kBins / kPartThreads;
+        unsigned long long w[kPer];
+        uint64_t z = 0, total;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            w[i] = state.bins[threadIdx.x * kPer + i];
+            z += w[i];
+        }
+        auto weight = [&](int i) -> uint64_t {
+            uint64_t v = 0;
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) v = (i & (kPer - 1)) == j ? w[j] : v;
+            return v;
+        };
+        block_scan<kPartThreads>(z, total);
+        const uint64_t target = draw == Draw::kTopK
+            ? uint64_t(k - 1)
+            : static_cast<uint64_t>(static_cast<double>(p) * static_cast<double>(total));
+        rest = target - first_over<kPartThreads>(kBins, kPer, target, cut, weight);
+        // Top-k beyond the bins' range: the whole row decides. (Top-p always
+        // finds its bin unless the target rounds to the whole mass: then
+        // everything is kept.)
+        whole = draw == Draw::kTopK && cut == kBins;
     }
-    auto in_k = [&](int64_t i) {
-        return kcut.all || kept(kcut, fkey(score_of(row, i, ctx)), i);
-    };
+    if (span == 0 && threadIdx.x == 0) {
+        state.rest = rest;
+        state.whole = whole;
+    }
+    if (whole) return;
 
-    Cut pcut{0u, 0, true};
-    if (p < 1.f) {
-        // Z = total mass of the top-k candidates (the softmax denominator).
-        __shared__ unsigned long long s_z;
-        if (threadIdx.x == 0) s_z = 0;
+    float best = -INFINITY;
+    int64_t bi = INT64_MAX;
+    const int64_t begin = int64_t(span) * kPartSpan;
+    const bool gather_all = draw == Draw::kTopK;  // every candidate into the list
+    uint4 words{};
+    int64_t held = -1;  // Philox block in `words`
+    for_span<T, VEC>(row, begin, min(vocab, begin + kPartSpan), [&](int64_t i, float x) {
+        const float s = (x - ctx.mx) / temp;
+        const int b = cut == kBins ? -1 : bin_of(s);
+        if (b > cut) return;
+        if (gather_all || b == cut) {
+            const uint32_t at = atomicAdd(&s_listed, 1u);
+            if (at < uint32_t(kListCap))
+                listed[at] = (static_cast<unsigned long long>(fkey(s)) << 32) |
+                             (0xffffffffu - static_cast<uint32_t>(i));
+            return;
+        }
+        if (held != (i >> 2)) {
+            held = i >> 2;
+            words = noise.block(i);
+        }
+        const int e = int(i & 3);
+        const float g = race_value(s, e == 0 ? words.x : e == 1 ? words.y
+                                                       : e == 2 ? words.z : words.w);
+        if (better(g, i, best, bi)) { best = g; bi = i; }
+    });
+    block_argmax_w<kPartThreads / 64>(best, bi);
+    if (threadIdx.x == 0) {
+        races[blockIdx.x] = ArgPart{best, bi == INT64_MAX ? -1 : int32_t(bi)};
+        s_at = s_listed ? atomicAdd(&state.listed, s_listed) : 0;
+    }
+    __syncthreads();
+    if (s_at + s_listed <= uint32_t(kListCap))  // else the row is drawn whole
+        for (uint32_t i = threadIdx.x; i < s_listed; i += kPartThreads)
+            state.list[s_at + i] = listed[i];
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+finish_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
+              const float* __restrict__ temperature, const int64_t* __restrict__ top_k,
+              const float* __restrict__ top_p, const int64_t* __restrict__ seeds,
+              const int64_t* __restrict__ counters, int64_t* __restrict__ out,
+              const ArgPart* __restrict__ parts, int nparts,
+              const RowState* __restrict__ states, const ArgPart* __restrict__ races) {
+    __shared__ unsigned long long order[kListCap];
+    const int r = blockIdx.x;
+    const float temp = temperature[r];
+    if (!(temp > 0.f)) return;
+    const RowState& state = states[r];
+    const int64_t k = top_k[r];
+    const float p = top_p[r];
+    const Noise noise = noise_of(seeds[r], counters[r]);
+    const uint32_t n = state.listed;
+    if (state.whole || n > uint32_t(kListCap)) {
+        const RowCtx ctx{row_max(parts + int64_t(r) * nparts, nparts).v, temp};
+        const int64_t token = sample_row<T, kThreads>(logits + int64_t(r) * stride, vocab, ctx, k,
+                                                      p, noise);
+        if (threadIdx.x == 0) out[r] = token;
+        return;
+    }
+    float best = -INFINITY;
+    int64_t bi = INT64_MAX;
+    for (int i = threadIdx.x; i < nparts; i += kThreads) {
+        const ArgPart q = races[int64_t(r) * nparts + i];
+        if (q.i >= 0 && better(q.v, q.i, best, bi)) { best = q.v; bi = q.i; }
+    }
+    if (n > 0) {
+        // Descending (key, then ascending index) order: a bitonic sort in
+        // LDS. Steps of up to 64 stay inside the 128 entries that a wave
+        // owns in all of them, so only the wider ones need the workgroup's
+        // barrier: at 1024 entries 6 of 55 steps.
+        int m = 2;
+        while (m < int(n)) m *= 2;
+        for (int i = threadIdx.x; i < m; i += kThreads)
+            order[i] = i < int(n) ? state.list[i] : 0ull;
         __syncthreads();
-        unsigned long long z = 0;
-        for (int64_t i = threadIdx.x; i < vocab; i += kThreads)
-            if (in_k(i)) z += mass_of(score_of(row, i, ctx));
-        atomicAdd(&s_z, z);
+        for (int size = 2; size <= m; size <<= 1)
+            for (int step = size >> 1; step > 0; step >>= 1) {
+                for (int t = threadIdx.x; t < m / 2; t += kThreads) {
+                    const int i = 2 * t - (t & (step - 1)), j = i + step;
+                    const unsigned long long a = order[i], b = order[j];
+                    if ((a < b) == ((i & size) == 0)) {
+                        order[i] = b;
+                        order[j] = a;
+                    }
+                }
+                const int next = step > 1 ? step >> 1 : size;
+                if (step > 64 || next > 64) {
+                    __syncthreads();
+                } else {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+            }
         __syncthreads();
-        const uint64_t target = static_cast<uint64_t>(static_cast<double>(p) *
-                                                      static_cast<double>(s_z));
-        pcut = radix_cut<T, true>(row, vocab, ctx, target, in_k);
+        auto mass = [&](int i) { return mass_of(key_value(uint32_t(order[i] >> 32))); };
+        const bool counted = k > 0 && k < vocab;  // the list holds every top-k candidate
+        int keep = counted ? int(k) : int(n);
+        if (p < 1.f) {
+            uint64_t rest = state.rest;
+            if (counted) {
+                uint64_t z = 0, total;
+                for (int i = threadIdx.x; i < keep; i += kThreads) z += mass(i);
+                block_scan<kThreads>(z, total);
+                rest = static_cast<uint64_t>(static_cast<double>(p) * static_cast<double>(total));
+            }
+            int pos;
+            first_over<kThreads>(keep, (keep + kThreads - 1) / kThreads, rest, pos, mass);
+            keep = min(keep, pos + 1);
+        }
+        for (int t = threadIdx.x; t < keep; t += kThreads) {
+            const int64_t i = int64_t(0xffffffffu - static_cast<uint32_t>(order[t]));
+            const float g = race_value(key_value(uint32_t(order[t] >> 32)), noise.bits(i));
+            if (better(g, i, best, bi)) { best = g; bi = i; }
+        }
     }
-
-    // Exponential race over the kept set: argmax s_i - log(E_i).
-    const uint2 key = make_uint2(static_cast<uint32_t>(seeds[r]),
-                                 static_cast<uint32_t>(uint64_t(seeds[r]) >> 32));
-    const uint64_t step = static_cast<uint64_t>(counters[r]);
-    float bv = -INFINITY;
-    int64_t bidx = INT64_MAX;
-    for (int64_t i = threadIdx.x; i < vocab; i += kThreads) {
-        const float s = score_of(row, i, ctx);
-        const uint32_t kk = fkey(s);
-        if (!kcut.all && !kept(kcut, kk, i)) continue;
-        if (!pcut.all && !kept(pcut, kk, i)) continue;
-        const uint4 rnd4 = philox4x32_10(
-            make_uint4(static_cast<uint32_t>(i >> 2), static_cast<uint32_t>(i >> 34),
-                       static_cast<uint32_t>(step), static_cast<uint32_t>(step >> 32)),
-            key);
-        const int lane4 = int(i & 3);
-        const uint32_t bits = lane4 == 0 ? rnd4.x : lane4 == 1 ? rnd4.y
-                            : lane4 == 2 ? rnd4.z : rnd4.w;
-        const float u = (float(bits >> 8) + 0.5f) * (1.0f / 16777216.0f);
-        const float e = -logf(u);
-        const float g = s - logf(e);
-        if (better(g, i, bv, bidx)) { bv = g; bidx = i; }
-    }
-    block_argmax(bv, bidx);
-    if (threadIdx.x == 0) out[r] = bidx;
+    block_argmax_w<kWaves>(best, bi);
+    if (threadIdx.x == 0) out[r] = bi;
 }
 
 template <typename T, bool VEC>
@@ -502,7 +892,7 @@ argmax_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
     float best = -INFINITY;
     int64_t bi = INT64_MAX;
     thread_argmax<T, VEC>(row, vocab, best, bi);
-    block_argmax(best, bi);
+    block_argmax_w<kWaves>(best, bi);
     if (threadIdx.x == 0) out[blockIdx.x] = bi;
 }
 
@@ -542,6 +932,12 @@ extern "C" int64_t tvllm_sample_workspace_size(int64_t rows, int64_t vocab) {
     return rows * ((vocab + kPartSpan - 1) / kPartSpan) * int64_t(sizeof(ArgPart));
 }
 
+extern "C" int64_t tvllm_sample_split_workspace_size(int64_t rows, int64_t vocab) {
+    // Each row's bins and list, and two (value, index) partials per span.
+    if (rows <= 0 || vocab <= 0) return 0;
+    return rows * int64_t(sizeof(RowState)) + 2 * tvllm_sample_workspace_size(rows, vocab);
+}
+
 extern "C" int tvllm_sample(const void* logits, int64_t rows, int64_t vocab,
                             int64_t row_stride, const float* temperature,
                             const int64_t* top_k, const float* top_p,
@@ -558,26 +954,47 @@ extern "C" int tvllm_sample(const void* logits, int64_t rows, int64_t vocab,
     TVLLM_CHECK(workspace_bytes >= 0 && (workspace_bytes == 0 || workspace != nullptr),
                 "sample: null workspace");
     hipStream_t s = as_hip(stream);
-    // With a workspace of tvllm_sample_workspace_size bytes the row scan is
-    // split over spans (argmax_part_kernel); without one each row's
-    // workgroup scans it alone.
+    // A workspace of tvllm_sample_split_workspace_size bytes spreads every
+    // pass over spans, one of tvllm_sample_workspace_size bytes the search for
+    // the row maximum only; without one each row's workgroup draws alone.
     const int64_t nparts = (vocab + kPartSpan - 1) / kPartSpan;
-    const bool split = workspace_bytes >= tvllm_sample_workspace_size(rows, vocab) &&
-                       aligned16(workspace) && rows * nparts <= INT32_MAX;
-    ArgPart* parts = split ? static_cast<ArgPart*>(workspace) : nullptr;
+    const bool fits = aligned16(workspace) && rows * nparts <= INT32_MAX;
+    const bool split = fits && workspace_bytes >= tvllm_sample_split_workspace_size(rows, vocab);
+    const bool scan = fits && workspace_bytes >= tvllm_sample_workspace_size(rows, vocab);
+    RowState* const states = split ? static_cast<RowState*>(workspace) : nullptr;
+    ArgPart* const parts = split ? reinterpret_cast<ArgPart*>(states + rows)
+                                 : scan ? static_cast<ArgPart*>(workspace) : nullptr;
     return dispatch_float(dtype, [&]<int DT>() {
         using T = typename Elem<DT>::T;
         const bool vec = sizeof(T) == 2 && row_stride % 8 == 0 && aligned16(logits);
         auto go = [&]<bool V>() {
-            if (split) {
-                argmax_part_kernel<T, V><<<int(rows * nparts), kPartThreads, 0, s>>>(
-                    static_cast<const T*>(logits), vocab, row_stride, int(nparts), parts);
+            const T* const x = static_cast<const T*>(logits);
+            const int grid = int(rows * nparts), np = int(nparts);
+            if (parts != nullptr) {
+                argmax_part_kernel<T, V><<<grid, kPartThreads, 0, s>>>(x, vocab, row_stride, np,
+                                                                       temperature, parts, states);
                 const int status = launch_status("sample");
                 if (status != TVLLM_OK) return status;
             }
-            sample_kernel<T, V><<<int(rows), kThreads, 0, s>>>(
-                static_cast<const T*>(logits), vocab, row_stride, temperature, top_k,
-                top_p, seeds, counters, out, parts, int(nparts));
+            if (!split) {
+                sample_kernel<T, V><<<int(rows), kThreads, 0, s>>>(
+                    x, vocab, row_stride, temperature, top_k, top_p, seeds, counters, out, parts,
+                    np);
+                return launch_status("sample");
+            }
+            bins_kernel<T, V><<<grid, kPartThreads, 0, s>>>(x, vocab, row_stride, temperature, top_k,
+                                                            top_p, out, parts, np, states);
+            int status = launch_status("sample");
+            if (status != TVLLM_OK) return status;
+            ArgPart* const races = parts + rows * nparts;
+            race_kernel<T, V><<<grid, kPartThreads, 0, s>>>(x, vocab, row_stride, temperature, top_k,
+                                                            top_p, seeds, counters, parts, np,
+                                                            states, races);
+            status = launch_status("sample");
+            if (status != TVLLM_OK) return status;
+            finish_kernel<T><<<int(rows), kThreads, 0, s>>>(x, vocab, row_stride, temperature, top_k,
+                                                            top_p, seeds, counters, out, parts, np,
+                                                            states, races);
             return launch_status("sample");
         };
         if constexpr (sizeof(T) == 2) {

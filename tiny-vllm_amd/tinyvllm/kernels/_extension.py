@@ -64,6 +64,7 @@ _SIGNATURES: dict[str, tuple[type, list[type]]] = {
                                   _INT, _INT, _F32, _F32, _P]),
     "tvllm_argmax": (_INT, [_P, _I64, _I64, _I64, _P, _INT, _P]),
     "tvllm_sample_workspace_size": (_I64, [_I64, _I64]),
+    "tvllm_sample_split_workspace_size": (_I64, [_I64, _I64]),
     "tvllm_sample": (_INT, [_P, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P,
                             _I64, _INT, _P]),
     "tvllm_resolve_tokens": (_INT, [_P, _P, _P, _I64, _I64, _P]),

@@ -62,9 +62,9 @@ def sample(
     if out is None:
         out = torch.empty(rows, dtype=torch.long, device=device)
     if rows:
-        # Per-span argmax partials: the row scan is spread over many
-        # workgroups (an allocation from torch's pool, graph-capturable).
-        size = lib.tvllm_sample_workspace_size(rows, vocab)
+        # Each row's passes are spread over many workgroups (an allocation
+        # from torch's pool, graph-capturable).
+        size = lib.tvllm_sample_split_workspace_size(rows, vocab)
         workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
         check(lib.tvllm_sample(
             logits.data_ptr(), rows, vocab, logits.stride(0), temperature.data_ptr(),
