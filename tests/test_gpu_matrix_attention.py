@@ -1,0 +1,112 @@
+"""The matrix-core kernels of head dims 32, 64 and 256 (and 128 for groups
+above 16): decode and prefill at the edges of their row tiles (16 rows, 64 and
+128 rows), key chunks (32 and 64 keys) and key splits, against the oracle; an
+infinity in V; and queries and outputs without vector alignment."""
+import math
+
+import pytest
+import torch
+
+from helpers import assert_bf16_close
+from oracle import attention as OA
+from test_gpu_fp8 import _fp8_cache
+from test_gpu_kernels import _Cache
+
+pytestmark = pytest.mark.gpu
+
+
+def _pool(g, contexts, bs=16):
+    pages = [math.ceil(n / bs) for n in contexts]
+    perm = torch.randperm(sum(pages) + 3, generator=g)
+    offsets = torch.tensor([0] + pages).cumsum(0)
+    return sum(pages) + 3, perm[:sum(pages)], offsets
+
+
+def _setup(g, contexts, kv_heads, dim, dtype, fp8, device, layout):
+    pool, blocks, offsets = _pool(g, contexts)
+    k = torch.randn(pool * 16, kv_heads, dim, generator=g)
+    v = torch.randn(pool * 16, kv_heads, dim, generator=g)
+    if fp8:
+        return (*_fp8_cache(k * 0.5, v * 2, 16, device, 0.5, 2.0, layout), blocks, offsets)
+    k, v = k.to(dtype), v.to(dtype)
+    return _Cache(k.to(device), v.to(device), 16, layout=layout), k, v, blocks, offsets
+
+
+def _prefill(device, q, cache, k, v, blocks, offsets, queries, contexts, dim, pad=0):
+    from tinyvllm.kernels.paged_prefill import paged_prefill_attention
+    from tinyvllm.runtime.contracts import MultiQueryMetadata
+
+    starts = torch.tensor([0] + queries).cumsum(0)
+    lengths = torch.tensor(contexts)
+    meta = MultiQueryMetadata(starts.to(device), blocks.to(device), offsets.to(device),
+                              lengths.to(device), max(queries))
+    wide = torch.zeros(*q.shape[:2], dim + pad, dtype=q.dtype, device=device)
+    qd = wide[..., pad:]
+    qd.copy_(q)
+    out = torch.zeros_like(wide)[..., pad:]
+    paged_prefill_attention(qd, cache, 0, meta, out, scale=dim ** -0.5)
+    expect = torch.zeros(q.shape, dtype=q.dtype)
+    OA.prefill_attention(q, k, v, starts, blocks, offsets, lengths, 16, dim ** -0.5, expect)
+    return out.cpu(), expect
+
+
+@pytest.mark.parametrize("dim,dtype,fp8", [(32, torch.bfloat16, False), (64, torch.float16, False),
+                                           (64, torch.bfloat16, True), (256, torch.bfloat16, False),
+                                           (256, torch.float16, True)])
+@pytest.mark.parametrize("kv_heads,group,items", [
+    (2, 4, [(5, 5), (8, 40), (9, 9), (1, 64)]),               # up to 36 rows: both kernels' side
+    (1, 2, [(8, 31), (16, 33)]),                              # 32 rows at most: 16-row groups
+    (1, 1, [(64, 64), (65, 97), (63, 127), (129, 400)]),      # 64-row tiles
+    (8, 8, [(77, 200)] * 5 + [(2, 65), (40, 40)]),            # 128-row tiles (256+ workgroups)
+])
+def test_prefill_tiles_match_oracle(device, dim, dtype, fp8, kv_heads, group, items):
+    g = torch.Generator().manual_seed(dim + group)
+    if kv_heads == 8:
+        items = items * 2
+    queries, contexts = [list(x) for x in zip(*items)]
+    cache, k, v, blocks, offsets = _setup(g, contexts, kv_heads, dim, dtype, fp8, device,
+                                          "head_major" if group == 4 else "token_major")
+    q = torch.randn(sum(queries), kv_heads * group, dim, generator=g).to(dtype)
+    out, expect = _prefill(device, q, cache, k, v, blocks, offsets, queries, contexts, dim)
+    assert_bf16_close(out, expect)
+
+
+@pytest.mark.parametrize("dim,pad", [(64, 1), (256, 4), (32, 2)])
+def test_unaligned_query_and_output_rows(device, dim, pad):
+    g = torch.Generator().manual_seed(dim)
+    queries, contexts = [50, 3], [90, 3]
+    cache, k, v, blocks, offsets = _setup(g, contexts, 2, dim, torch.bfloat16, False, device,
+                                          "token_major")
+    q = torch.randn(53, 4, dim, generator=g).to(torch.bfloat16)
+    out, expect = _prefill(device, q, cache, k, v, blocks, offsets, queries, contexts, dim, pad)
+    assert_bf16_close(out, expect)
+
+
+@pytest.mark.parametrize("dim,group", [(32, 2), (64, 4), (256, 3), (128, 20)])
+@pytest.mark.parametrize("longest", [30, 5000])
+def test_decode_with_an_infinite_value(device, dim, group, longest):
+    """Rows whose V holds an infinity give that infinity (their weights there
+    are positive); the other rows and dims are untouched by it."""
+    from tinyvllm.kernels.paged_decode import paged_decode_attention
+    from tinyvllm.runtime.contracts import SingleQueryMetadata
+
+    g = torch.Generator().manual_seed(dim)
+    contexts = [longest, 17, 64]
+    cache, k, v, blocks, offsets = _setup(g, contexts, 2, dim, torch.bfloat16, False, device,
+                                          "token_major")
+    slot = int(blocks[(contexts[0] - 1) // 16]) * 16 + (contexts[0] - 1) % 16
+    for t in (v, cache.value[0]):
+        t[slot, 1, 3] = float("inf")
+    q = torch.randn(3, 2 * group, dim, generator=g).to(torch.bfloat16)
+    rows, lengths = torch.arange(3), torch.tensor(contexts)
+    meta = SingleQueryMetadata(rows.to(device), blocks.to(device), offsets.to(device),
+                               lengths.to(device), longest)
+    out = torch.zeros(q.shape, dtype=q.dtype, device=device)
+    paged_decode_attention(q.to(device), cache, 0, meta, out, scale=dim ** -0.5)
+    expect = torch.zeros(q.shape, dtype=q.dtype)
+    OA.decode_attention(q, k, v, rows, blocks, offsets, lengths, 16, dim ** -0.5, expect)
+    out = out.cpu()
+    assert bool((expect[0, group:, 3] == float("inf")).all())
+    assert torch.equal(torch.isinf(out), torch.isinf(expect))
+    finite = torch.isfinite(expect)
+    assert_bf16_close(out[finite], expect[finite])

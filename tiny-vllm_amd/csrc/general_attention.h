@@ -40,6 +40,7 @@ struct GeneralAttention {
     int64_t splits, split_keys;
     float* part_o;   // [num_items][heads][splits][head_dim]
     float* part_ml;  // [num_items][heads][splits][2]: (max, sum) in base 2
+    bool q_vec, out_vec;  // query rows in 16-byte pieces, output rows in 8-byte ones
 };
 
 // Grid-level key splits of a decode launch of the general kernel (1: none):

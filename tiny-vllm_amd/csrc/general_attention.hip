@@ -8,16 +8,17 @@
 // 176-214). Output = softmax(scale * q.K^T) V over each row's cached tokens
 // in logical order (a padded decode row of length 0 gives zeros).
 //
-// Design: one wave per (query token, KV head, group of up to 16 query heads
-// of that KV head), so the query heads of a KV head share every K/V load.
-// The wave walks its keys in chunks of 64: lane j scores key j of the chunk
-// against all of the wave's heads (the query rows sit in LDS, read as
-// broadcasts), the online softmax runs per head across the wave, and P.V
-// runs with the lanes over the head dims (lane l: dims l, l + 64, ...), the
-// chunk's probabilities read back from LDS. Everything is fp32 (the query
-// pre-multiplied by scale * log2(e)); no matrix cores - these shapes are
-// outside every benchmark configuration, and the fp32 path is exact enough
-// to need no fallback of its own.
+// Head dims 32, 64, 128 and 256 with vector-aligned cache rows run on the
+// matrix cores (rows_attention_kernel for few query rows, decode above all;
+// tiles_attention_kernel for prefill chunks). Everything else - other head
+// dims, unaligned rows - takes general_attention_kernel: one wave per (query
+// token, KV head, group of up to 16 query heads of that KV head), so the
+// query heads of a KV head share every K/V load. The wave walks its keys in
+// chunks of 64: lane j scores key j of the chunk against all of the wave's
+// heads (the query rows sit in LDS, read as broadcasts), the online softmax
+// runs per head across the wave, and P.V runs with the lanes over the head
+// dims (lane l: dims l, l + 64, ...), the chunk's probabilities read back
+// from LDS. That kernel is fp32 throughout, without matrix cores.
 #include "general_attention.h"
 
 #include <algorithm>
@@ -30,14 +31,6 @@ constexpr int GH = 16;     // query heads per wave
 constexpr int DMAX = 256;  // largest head dim
 constexpr float kLog2eG = 1.4426950408889634f;
 constexpr int kRowWaves = 4;  // waves per workgroup of the row-tiled kernel
-
-// Orders one wave's LDS writes before its own later reads (no other wave is
-// involved): a compiler barrier - the wave's LDS operations run in order.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Eight elements of a cache row starting at element e (FP8: bytes), as
 // floats; elements at or past `left` read as 0.
@@ -213,43 +206,231 @@ __global__ void __launch_bounds__(64) general_attention_kernel(GeneralAttention 
     }
 }
 
-// The reference's head dims (32, 64, 128, 256) with vector-aligned rows.
-// A workgroup serves up to 16 (query token, query head) rows of one KV head:
-// one query's group of heads (up to 16), or for groups below 16 several
-// consecutive queries of one prefill item, each row with its own causal
-// bound. Its four waves take interleaved chunks of KPC keys: LPK lanes share
-// a key (each holds EPL <= 64 of its dims), K and V pieces of the whole
-// chunk are loaded at once and the wave's next chunk is in flight during
-// this chunk's P.V; V is staged in the wave's own LDS buffer (FP8 widened
-// exactly to T) for P.V with the lanes over the dims, each key's
-// probabilities broadcast from the lanes that scored it. The waves' (max,
-// sum, accumulator) merge through LDS at the end.
-template <typename T, bool F8, int D>
-__global__ void __launch_bounds__(64 * kRowWaves) rows_attention_kernel(GeneralAttention a) {
-    constexpr int LPK = D > 64 ? D / 64 : 1;  // lanes per key
-    constexpr int EPL = D / LPK;               // elements per lane
-    constexpr int KPC = 64 / LPK;              // keys per chunk
-    constexpr int NV = EPL / 8;                // 8-element pieces per lane
-    constexpr int DI = (D + 63) / 64;          // output dims per lane
-    using Piece = std::conditional_t<F8, uint2, uint4>;  // native vectors: kept in registers
-    constexpr int NW = kRowWaves;
-    // LDS: the rows' queries and each wave's staged V chunk; after the key
-    // loop the same bytes hold waves 1..NW-1's partial results for the merge.
-    // Staged V rows are padded by 16 bytes, so the lanes' 16-byte row writes
-    // (one key per lane, rows D * 2 bytes apart) spread over the LDS banks.
-    constexpr int VS = D + 8;  // staged V row stride (elements)
-    constexpr int kMain = GH * D * 4 + NW * KPC * VS * 2;
-    constexpr int kMerge = (NW - 1) * GH * (D + 2) * 4;
-    __shared__ __align__(16) unsigned char smem[kMain > kMerge ? kMain : kMerge];
-    float (*const qs)[D] = reinterpret_cast<float (*)[D]>(smem);
-    const int wave = threadIdx.x >> 6;
-    U16x8 (*const vs)[VS / 8] =
-        reinterpret_cast<U16x8 (*)[VS / 8]>(smem + GH * D * 4 + wave * KPC * VS * 2);
+// ------------------------------------------------- matrix-core kernels ----
+// The reference's head dims (32, 64, 128, 256) with vector-aligned cache
+// rows, on 16x16x32 MFMAs. Both kernels compute S^T = K Q^T (a lane holds the
+// scores of query row lane % 16) and O^T = V^T P^T, whose B operand is exactly
+// the lane's own scores and whose accumulators belong to the same query row:
+// the softmax, its rescaling and the output are lane-local, with two shuffles
+// per reduction over the keys. The k index of P.V runs over 32 keys in the
+// order (quad, tile, i) of the score layout: key 16 * tile + 4 * quad + i at
+// k = 8 * quad + 4 * tile + i.
+//
+// Precision: Q.K^T takes the stored 16-bit values (their products are exact
+// in fp32) and the scale is applied in fp32; P enters P.V as two terms of the
+// storage type (P rounded, and the rounded remainder: 16 bits for bf16, 22
+// for fp16), the denominator sums the unrounded P, accumulation is fp32.
 
+typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 gf16x8 __attribute__((ext_vector_type(8)));
+typedef float gf32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+__device__ __forceinline__ gf32x4 mfma32(const U16x8& a, const U16x8& b, gf32x4 c) {
+    if constexpr (std::is_same_v<T, __bf16>) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, a),
+                                                       __builtin_bit_cast(gbf16x8, b), c, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gf16x8, a),
+                                                      __builtin_bit_cast(gf16x8, b), c, 0, 0, 0);
+    }
+}
+
+// Elements 2 * w and 2 * w + 1 of words a (first) and b: the even (or odd)
+// elements of the two side by side.
+__device__ __forceinline__ uint32_t pair_lo(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_perm(b, a, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t pair_hi(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
+// Two FP8 elements (the low or high half of w) widened exactly to one word of T.
+template <typename T, bool HI>
+__device__ __forceinline__ uint32_t widen2(uint32_t w) {
+    if constexpr (std::is_same_v<T, __bf16>) {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, HI));
+    } else {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, HI));
+    }
+}
+
+// P of a 32-key group (8 scores' weights, k order) as the two B operands.
+template <typename T>
+__device__ __forceinline__ void split_p(const float (&p)[8], U16x8& hi, U16x8& lo) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        hi.w[w] = pack2<T>(p[2 * w], p[2 * w + 1]);
+        lo.w[w] = pack2<T>(p[2 * w] - half_lo<T>(hi.w[w]), p[2 * w + 1] - half_hi<T>(hi.w[w]));
+    }
+}
+
+// Max / sum over the four quads that share a query row.
+__device__ __forceinline__ float quad_max(float v) {
+    v = fmaxf(v, __shfl_xor(v, 16, 64));
+    return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+}
+
+// The online softmax of one step: x holds the lane's scores (base 2, masked
+// ones -inf) and becomes the weights 2^(x - m). The reference m follows the
+// running maximum only once some row of the wave exceeds it by 8: until then
+// the weights stay below 2^8 and nothing needs rescaling. Returns whether it
+// moved; `alpha` is then the factor of what was summed before. Rows with no
+// key yet keep m = -inf and weights 0.
+template <int N>
+__device__ __forceinline__ bool softmax_step(float (&x)[N], float& m, float& l, float& alpha) {
+    float top = x[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i) top = fmaxf(top, x[i]);
+    top = quad_max(top);
+    const bool moved = __any(top > m + 8.f);  // m = -inf: any key at all
+    if (moved) {
+        const float mn = fmaxf(m, top);
+        alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
+        l *= alpha;
+    }
+    const float base = m == -INFINITY ? 0.f : m;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        x[i] = __builtin_amdgcn_exp2f(x[i] - base);
+        sum += x[i];
+    }
+    l += sum;  // this lane's share of the denominator
+    return moved;
+}
+
+// Eight elements of a query row as an operand piece.
+template <typename T>
+__device__ __forceinline__ U16x8 load_query(const T* p, bool vec) {
+    if (vec) return *reinterpret_cast<const U16x8*>(p);
+    U16x8 r;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        r.w[w] = uint32_t(__builtin_bit_cast(uint16_t, p[2 * w])) |
+                 uint32_t(__builtin_bit_cast(uint16_t, p[2 * w + 1])) << 16;
+    return r;
+}
+
+// Writes n (a multiple of 4) consecutive elements, rounded to T.
+template <typename T, int N>
+__device__ __forceinline__ void store_row(T* o, const float (&x)[N], float inv, bool vec) {
+    if (vec) {
+#pragma unroll
+        for (int i = 0; i < N; i += 4)
+            *reinterpret_cast<uint2*>(o + i) =
+                make_uint2(pack2<T>(x[i] * inv, x[i + 1] * inv),
+                           pack2<T>(x[i + 2] * inv, x[i + 3] * inv));
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = static_cast<T>(x[i] * inv);
+    }
+}
+
+// One row by one wave in plain fp32 over keys [k_begin, k_end): the answer for
+// a row whose accumulators end non-finite. An infinity in V meets zero terms
+// above (the remainder of an exact P, masked or repeated keys), and 0 * inf is
+// NaN where the sum over the row's own keys may be infinite. Lane l scores
+// key l of each 64, and holds the output dims l, l + 64, ...
+template <typename T, bool F8, int D>
+__device__ __forceinline__ void exact_row(const GeneralAttention& a, const T* q,
+                                                    int kvh, int64_t table, int64_t k_begin,
+                                                    int64_t k_end, float& m, float& l,
+                                                    float (&acc)[(D + 63) / 64]) {
+    constexpr int DI = (D + 63) / 64;
     const int lane = threadIdx.x & 63;
+    const float qscale = a.scale * kLog2eG * a.k_scale;
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < DI; ++i) acc[i] = 0.f;
+    for (int64_t t0 = k_begin; t0 < k_end; t0 += 64) {
+        const int64_t t = min(t0 + lane, k_end - 1);
+        const int64_t page = t / a.block_size;
+        const int64_t base = (a.blocks[table + page] * a.block_size + (t - page * a.block_size)) *
+                                 a.css + int64_t(kvh) * a.chs;
+        float s = 0.f;
+        for (int d = 0; d < D; d += 8) {
+            float x[8];
+            load8<T, F8, true>(a.k, base + d, 8, x);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s = fmaf(to_f<T>(q[d + i]) * qscale, x[i], s);
+        }
+        if (t0 + lane >= k_end) s = -INFINITY;
+        const float mn = fmaxf(m, wave_max(s));
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        const float alpha = exp2f(m - ref);
+        const float p = exp2f(s - ref);
+        l = l * alpha + wave_sum(p);
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < DI; ++i) acc[i] *= alpha;
+        const int n = int(min<int64_t>(64, k_end - t0));
+        for (int j = 0; j < n; ++j) {
+            const float pj = __shfl(p, j, 64);
+            const int64_t row = int64_t(uint64_t(uint32_t(__shfl(int(uint64_t(base) >> 32), j, 64)))
+                                            << 32 |
+                                        uint32_t(__shfl(int(uint32_t(base)), j, 64)));
+#pragma unroll
+            for (int i = 0; i < DI; ++i) {
+                const int d = lane + 64 * i;
+                if (d < D) acc[i] = fmaf(pj, load1<T, F8>(a.v, row + d), acc[i]);
+            }
+        }
+    }
+}
+
+template <int N>
+__device__ __forceinline__ bool all_finite(const float (&x)[N], float den) {
+    bool ok = den < INFINITY;  // false for NaN too
+#pragma unroll
+    for (int i = 0; i < N; ++i) ok = ok && fabsf(x[i]) < INFINITY;
+    return ok;
+}
+
+// Few query rows against many keys: decode, and prefill calls of a few
+// queries. A workgroup serves up to 16 (query token, query head) rows of one
+// KV head: one query's group of heads (up to 16), or for groups below 16
+// several consecutive queries of one prefill item, each row with its own
+// causal bound. Its four waves take interleaved chunks of CH keys straight
+// from the cache into operand registers, with no LDS on the way: lane (col,
+// quad) holds the K pieces of key col as the A operand, and of V the dims
+// VE * col .. of the keys 4 * quad + i, which gathered by element (v_perm)
+// are the A operand of one MFMA per element. The next chunk's K loads are
+// issued right after Q.K^T, its V loads after P.V. The waves' (max, sum,
+// accumulator) merge through LDS at the end.
+//
+// Bound by the rate of its loads at many rows, by their latency along the
+// longest row at few. In us, against fp32 arithmetic on the vector units
+// (K and V broadcast to the query rows' lanes): 64 rows x 2048 tokens, 32
+// query and 8 KV heads of 64 167 -> 57 (4.7 TB/s of 128-byte pieces), of 256
+// 364 -> 177 (6.1 TB/s); 256 / 8 heads of 128 907 -> 158; 33 rows of 1-4096
+// tokens, heads of 64 165 -> 47. Two tiles per chunk rather than four
+// (142 registers, three waves per SIMD): 1-7 % at head dim 64.
+template <typename T, bool F8, int D>
+__global__ void __launch_bounds__(64 * kRowWaves)
+rows_attention_kernel(GeneralAttention a) {
+    constexpr int NT = 2;                // 16-key tiles per chunk
+    constexpr int CH = 16 * NT;
+    constexpr int KS = D / 32;           // Q.K^T steps
+    constexpr int VE = D / 16;           // dims per lane and key of V
+    constexpr int NW = kRowWaves;
+    constexpr int EB = F8 ? 1 : 2;       // cache bytes per element
+    constexpr int VW = VE / 2;           // V words per key, widened
+    __shared__ float part_acc[(NW - 1) * VE * 4 * 64];
+    __shared__ float part_ml[NW - 1][2][64];
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 15, quad = lane >> 4;
+
     const int group = a.heads / a.kv_heads;
-    const int hpq = group >= GH ? GH : group;   // heads per query in a wave
-    const int qpw = group >= GH ? 1 : GH / group;  // queries per wave
+    const int hpq = group >= GH ? GH : group;       // heads per query
+    const int qpw = group >= GH ? 1 : GH / group;   // queries per workgroup
     const int chunks = (group + GH - 1) / GH;
     const int64_t bx = blockIdx.x;
     const int hc = int(bx % chunks);
@@ -276,236 +457,540 @@ __global__ void __launch_bounds__(64 * kRowWaves) rows_attention_kernel(GeneralA
     const int hw = min(hpq, group - g0);
     const int nrows = int(nq) * hw;
     const int64_t ctx = a.lengths[item];
-    const int64_t first_end = ctx - qlen + q0 + 1;  // causal bound of the wave's first query
-    const int64_t kv_max = first_end + nq - 1;       // ... and of its last
-    const float qscale = a.scale * kLog2eG * a.k_scale;
-    const T* const q = static_cast<const T*>(a.q);
+    const int64_t first_end = ctx - qlen + q0 + 1;  // causal bound of the first query
+    const int64_t kv_max = first_end + nq - 1;       // ... and of the last
     T* const out = static_cast<T*>(a.out);
-    auto row_token = [&](int r) { return tok0 + r / hw; };
-    auto row_head = [&](int r) { return kvh * group + g0 + r % hw; };
     // Keys [k_begin, k_end) of this split (all of them when unsplit). The
     // last split also takes any keys past splits * split_keys (a row longer
     // than the max_context the plan was sized for): slow, never wrong.
     const int64_t k_begin = split * a.split_keys;
     const int64_t k_end = a.splits > 1 && split + 1 < a.splits
         ? min(kv_max, k_begin + a.split_keys) : kv_max;
-    auto part_index = [&](int r) { return (item * a.heads + row_head(r)) * a.splits + split; };
+    const int row = min(col, nrows - 1);  // this lane's query row
+    const int64_t token = tok0 + row / hw;
+    const int head = kvh * group + g0 + row % hw;
+    const int64_t part = (item * a.heads + head) * a.splits + split;
 
     if (a.splits > 1 && k_begin >= k_end) {  // no key of the row in this split
-        for (int r = threadIdx.x; r < nrows; r += 64 * NW) {
-            a.part_ml[2 * part_index(r)] = -INFINITY;  // the merge skips it
-            a.part_ml[2 * part_index(r) + 1] = 0.f;
+        if (wave == 0 && quad == 0 && col < nrows) {
+            a.part_ml[2 * part] = -INFINITY;  // the merge skips it
+            a.part_ml[2 * part + 1] = 0.f;
         }
         return;  // uniform per workgroup
     }
-
     if (kv_max <= 0) {  // no key for any row (a padded decode row): zeros, and
                         // no read of its block table, which may hold no entry
-        for (int r = 0; r < nrows; ++r)
-            for (int d = threadIdx.x; d < D; d += 64 * NW)
-                out[row_token(r) * a.ots + row_head(r) * a.ohs + d] = static_cast<T>(0.f);
+        for (int i = threadIdx.x; i < nrows * D; i += 64 * NW) {
+            const int r = i / D;
+            out[(tok0 + r / hw) * a.ots + (kvh * group + g0 + r % hw) * a.ohs + i % D] =
+                static_cast<T>(0.f);
+        }
         return;  // uniform per workgroup
     }
-    for (int r = 0; r < nrows; ++r)
-        for (int d = threadIdx.x; d < D; d += 64 * NW)
-            qs[r][d] = to_f<T>(q[row_token(r) * a.qts + row_head(r) * a.qhs + d]) * qscale;
-    __syncthreads();
-
-    float m[GH], l[GH], acc[GH][DI];
+    U16x8 qb[KS];
+    const T* const q = static_cast<const T*>(a.q) + token * a.qts + head * a.qhs + 8 * quad;
 #pragma unroll
-    for (int r = 0; r < GH; ++r) {
-        m[r] = -INFINITY;
-        l[r] = 0.f;
-#pragma unroll
-        for (int i = 0; i < DI; ++i) acc[r][i] = 0.f;
+    for (int s = 0; s < KS; ++s) {
+        qb[s] = load_query<T>(q + 32 * s, a.q_vec);
+        if (col >= nrows) qb[s] = U16x8{};
     }
-    const int64_t table = a.offsets[item];
-    const int bs = a.block_size;
-    const int kp = lane / LPK;    // the lane's key within a chunk
-    const int part = lane % LPK;  // ... and its share of the dims
-    const int64_t lane_off = int64_t(kvh) * a.chs + part * EPL;
+    // Keys this lane's row attends: none beyond the group's rows.
+    const int64_t bound = col < nrows ? min(first_end + row / hw, k_end) : 0;
+    const float qscale = a.scale * kLog2eG * a.k_scale;
 
-    struct Chunk {
-        Piece k[NV], v[NV];
+    const int64_t table = a.offsets[item];
+    const uint32_t bs = uint32_t(a.block_size);
+    const char* const kc = static_cast<const char*>(a.k) + int64_t(kvh) * a.chs * EB;
+    const char* const vc = static_cast<const char*>(a.v) + int64_t(kvh) * a.chs * EB;
+    // The cache row of chunk key t0 + lane % CH (past the end: the row's last
+    // key, a valid row that the mask drops), in two steps: its block id, whose
+    // load is issued a chunk ahead of its use, and its byte offset.
+    auto load_id = [&](int64_t t0) -> int64_t {
+        return a.blocks[table + uint32_t(min(t0 + lane % CH, kv_max - 1)) / bs];
     };
-    auto load_chunk = [&](int64_t t0) -> Chunk {
-        const int64_t t = max<int64_t>(min(t0 + kp, kv_max - 1), 0);  // a valid row
-        const int64_t page = t / bs;
-        const int64_t base = (a.blocks[table + page] * bs + (t - page * bs)) * a.css + lane_off;
-        Chunk c;
+    auto resolve = [&](int64_t t0, int64_t id) -> int64_t {
+        const uint32_t t = uint32_t(min(t0 + lane % CH, kv_max - 1));
+        return (id * bs + t % bs) * a.css * EB;
+    };
+    auto at = [&](int64_t off, int key) -> int64_t {
+        const uint32_t lo = uint32_t(__shfl(int(uint32_t(off)), key, 64));
+        const uint32_t hi = uint32_t(__shfl(int(uint32_t(uint64_t(off) >> 32)), key, 64));
+        return int64_t(uint64_t(hi) << 32 | lo);
+    };
+    using KPiece = std::conditional_t<F8, uint2, U16x8>;
+    KPiece kreg[NT][KS];
+    constexpr int VB = VE * EB;  // V bytes per lane and key
+    uint32_t vreg[NT][4][(VB + 3) / 4];
+    auto load_k = [&](int64_t off) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if constexpr (F8) {
-                c.k[v] = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(a.k) + base + 8 * v);
-                c.v[v] = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(a.v) + base + 8 * v);
-            } else {
-                c.k[v] = *reinterpret_cast<const uint4*>(static_cast<const T*>(a.k) + base + 8 * v);
-                c.v[v] = *reinterpret_cast<const uint4*>(static_cast<const T*>(a.v) + base + 8 * v);
-            }
+        for (int j = 0; j < NT; ++j) {
+            const char* const p = kc + at(off, 16 * j + col) + 8 * quad * EB;
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+                kreg[j][s] = *reinterpret_cast<const KPiece*>(p + 32 * s * EB);
         }
-        return c;
     };
+    auto load_v = [&](int64_t off) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const char* const p = vc + at(off, 16 * j + 4 * quad + i) + col * VB;
+                if constexpr (VB == 2) {
+                    vreg[j][i][0] = *reinterpret_cast<const uint16_t*>(p);
+                } else if constexpr (VB == 4) {
+                    vreg[j][i][0] = *reinterpret_cast<const uint32_t*>(p);
+                } else if constexpr (VB == 8) {
+                    const uint2 x = *reinterpret_cast<const uint2*>(p);
+                    vreg[j][i][0] = x.x;
+                    vreg[j][i][1] = x.y;
+                } else {
+#pragma unroll
+                    for (int w = 0; w < VB / 16; ++w) {
+                        const U16x8 x = *reinterpret_cast<const U16x8*>(p + 16 * w);
+#pragma unroll
+                        for (int y = 0; y < 4; ++y) vreg[j][i][4 * w + y] = x.w[y];
+                    }
+                }
+            }
+    };
+    // Word w (elements 2w, 2w + 1) of the lane's V piece of key (j, i), in T.
+    auto v_word = [&](int j, int i, int w) -> uint32_t {
+        if constexpr (F8) {
+            return (w & 1) ? widen2<T, true>(vreg[j][i][w / 2])
+                           : widen2<T, false>(vreg[j][i][w / 2]);
+        } else {
+            return vreg[j][i][w];
+        }
+    };
+
+    gf32x4 acc[VE];  // acc[e][v]: dim VE * (4 * quad + v) + e of the lane's row
+#pragma unroll
+    for (int e = 0; e < VE; ++e) acc[e] = gf32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
 
     // Wave w takes chunks w, w + NW, ... of the keys.
-    Chunk cur = load_chunk(k_begin + int64_t(wave) * KPC);
-    for (int64_t t0 = k_begin + int64_t(wave) * KPC; t0 < k_end; t0 += NW * KPC) {
-        // The chunk's V pieces into LDS, its K pieces unpacked to floats.
-        float x[NV][8];
+    int64_t t0 = k_begin + int64_t(wave) * CH;
+    if (t0 < k_end) {
+        constexpr int64_t kStep = NW * CH;
+        int64_t off = resolve(t0, load_id(t0));
+        int64_t id = load_id(t0 + kStep);
+        load_k(off);
+        load_v(off);
+        asm volatile("" ::: "memory");  // see below
+        for (; t0 < k_end; t0 += kStep) {
+            off = resolve(t0 + kStep, id);
+            id = load_id(t0 + 2 * kStep);
+            float x[4 * NT];
+            // Keys of the chunk from this quad's first on that the row sees.
+            const int left = int(max<int64_t>(min<int64_t>(bound - t0, CH), 0)) - 4 * quad;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if constexpr (F8) {
-                vs[kp][(part * EPL) / 8 + v] = fp8x8_widen<T>(cur.v[v]);  // exact in T
-                fp8x8_unpack(cur.k[v], x[v]);
-            } else {
-                vs[kp][(part * EPL) / 8 + v] = __builtin_bit_cast(U16x8, cur.v[v]);
-                unpack8<T>(__builtin_bit_cast(U16x8, cur.k[v]), x[v]);
-            }
-        }
-        float s[GH];
+            for (int j = 0; j < NT; ++j) {
+                gf32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < GH; ++r) {
-            s[r] = 0.f;
-            if (r < nrows) {  // uniform
-                float y = 0.f;
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    const int d = part * EPL + 8 * v;
-                    const float4 qa = *reinterpret_cast<const float4*>(&qs[r][d]);
-                    const float4 qb = *reinterpret_cast<const float4*>(&qs[r][d + 4]);
-                    y = fmaf(qa.x, x[v][0], y);
-                    y = fmaf(qa.y, x[v][1], y);
-                    y = fmaf(qa.z, x[v][2], y);
-                    y = fmaf(qa.w, x[v][3], y);
-                    y = fmaf(qb.x, x[v][4], y);
-                    y = fmaf(qb.y, x[v][5], y);
-                    y = fmaf(qb.z, x[v][6], y);
-                    y = fmaf(qb.w, x[v][7], y);
-                }
-                s[r] = y;
-            }
-        }
-        const int64_t key = t0 + kp;
-        float pr[GH];  // this lane's key's probability for each row
-#pragma unroll
-        for (int r = 0; r < GH; ++r) {
-            pr[r] = 0.f;
-            if (r >= nrows) continue;
-            float sr = s[r];
-            if constexpr (LPK > 1) sr += __shfl_xor(sr, 1, 64);
-            if constexpr (LPK > 2) sr += __shfl_xor(sr, 2, 64);
-            // Row r (query r / hw) sees keys below its own causal bound.
-            const float sg = key < first_end + r / hw && key < k_end ? sr : -INFINITY;
-            const float mn = fmaxf(m[r], wave_max(sg));
-            const float alpha = mn == -INFINITY ? 1.f : exp2f(m[r] - mn);
-            const float p = sg == -INFINITY ? 0.f : exp2f(sg - mn);
-            l[r] = l[r] * alpha + wave_sum(part == 0 ? p : 0.f);
-#pragma unroll
-            for (int i = 0; i < DI; ++i) acc[r][i] *= alpha;
-            m[r] = mn;
-            pr[r] = p;
-        }
-        wave_sync();  // the chunk's V rows are in LDS
-        // The next chunk's rows (past the end: clamped, valid rows, loaded
-        // unconditionally so the loaded registers are no loop-carried
-        // choice) are in flight during P.V.
-        cur = load_chunk(t0 + NW * KPC);
-        const int n = int(min<int64_t>(KPC, k_end - t0));
-        const uint16_t* const vrow = reinterpret_cast<const uint16_t*>(&vs[0][0]);
-        // Eight keys at a time: their V elements are read from LDS together,
-        // and each key's probabilities come from the lanes that scored it
-        // (a register broadcast, no LDS round trip).
-        for (int j0 = 0; j0 < n; j0 += 8) {
-            float vv[8][DI];
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj)
-#pragma unroll
-                for (int i = 0; i < DI; ++i) {
-                    const int d = lane + 64 * i;
-                    vv[jj][i] = (j0 + jj < n && d < D)
-                        ? to_f<T>(__builtin_bit_cast(T, vrow[(j0 + jj) * VS + d])) : 0.f;
+                for (int s = 0; s < KS; ++s) {
+                    if constexpr (F8) sc = mfma32<T>(fp8x8_widen<T>(kreg[j][s]), qb[s], sc);
+                    else sc = mfma32<T>(kreg[j][s], qb[s], sc);
                 }
 #pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                if (j0 + jj >= n) continue;  // uniform
+                for (int i = 0; i < 4; ++i)
+                    x[4 * j + i] = 16 * j + i < left ? sc[i] * qscale : -INFINITY;
+            }
+            load_k(off);
+            // The scheduler would gather V's operands ahead of these loads,
+            // and wait for V there.
+            __builtin_amdgcn_sched_barrier(0);
+            float alpha;
+            if (softmax_step(x, m, l, alpha)) {
 #pragma unroll
-                for (int r = 0; r < GH; ++r) {
-                    if (r >= nrows) continue;
-                    const float p = __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pr[r]),
-                                                         (j0 + jj) * LPK));
+                for (int e = 0; e < VE; ++e) acc[e] *= alpha;
+            }
 #pragma unroll
-                    for (int i = 0; i < DI; ++i) acc[r][i] = fmaf(p, vv[jj][i], acc[r][i]);
+            for (int g = 0; g < NT / 2; ++g) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[i] = x[8 * g + i];
+                U16x8 hi, lo;
+                split_p<T>(p, hi, lo);
+#pragma unroll
+                for (int w = 0; w < VW; ++w) {
+                    U16x8 even, odd;
+#pragma unroll
+                    for (int y = 0; y < 4; ++y) {
+                        const int j = 2 * g + y / 2, i = 2 * (y & 1);
+                        const uint32_t v0 = v_word(j, i, w), v1 = v_word(j, i + 1, w);
+                        even.w[y] = pair_lo(v0, v1);
+                        odd.w[y] = pair_hi(v0, v1);
+                    }
+                    acc[2 * w] = mfma32<T>(even, hi, acc[2 * w]);
+                    acc[2 * w + 1] = mfma32<T>(odd, hi, acc[2 * w + 1]);
+                    acc[2 * w] = mfma32<T>(even, lo, acc[2 * w]);
+                    acc[2 * w + 1] = mfma32<T>(odd, lo, acc[2 * w + 1]);
                 }
             }
+            load_v(off);
+            // Nothing is written; but a possible write keeps the compiler from
+            // turning the loaded values carried into the next iteration into
+            // loads there, right in front of their uses.
+            asm volatile("" ::: "memory");
         }
-        wave_sync();  // the wave's V buffer is rewritten by the next chunk
     }
+    l = quad_sum(l);
 
     // Merge the waves' partial results: out = sum_w 2^(m_w - M) acc_w /
     // sum_w 2^(m_w - M) l_w per row (M the largest m_w); a row with no key
     // in any wave gives zeros.
-    __syncthreads();  // every wave is past its last LDS read of qs and vs
-    float* const part_acc = reinterpret_cast<float*>(smem);          // [NW-1][GH][D]
-    float* const part_ml = part_acc + (NW - 1) * GH * D;             // [NW-1][GH][2]
     if (wave > 0) {
 #pragma unroll
-        for (int r = 0; r < GH; ++r) {
-            if (r >= nrows) continue;
-            float* const pa = part_acc + ((wave - 1) * GH + r) * D;
+        for (int e = 0; e < VE; ++e)
 #pragma unroll
-            for (int i = 0; i < DI; ++i) {
-                const int d = lane + 64 * i;
-                if (d < D) pa[d] = acc[r][i];
-            }
-            if (lane == 0) {
-                part_ml[((wave - 1) * GH + r) * 2] = m[r];
-                part_ml[((wave - 1) * GH + r) * 2 + 1] = l[r];
-            }
-        }
+            for (int v = 0; v < 4; ++v)
+                part_acc[((wave - 1) * VE * 4 + 4 * e + v) * 64 + lane] = acc[e][v];
+        part_ml[wave - 1][0][lane] = m;
+        part_ml[wave - 1][1][lane] = l;
     }
     __syncthreads();
     if (wave > 0) return;
+    float mx = m;
 #pragma unroll
-    for (int r = 0; r < GH; ++r) {
-        if (r >= nrows) continue;
-        float mx = m[r];
-        for (int w = 1; w < NW; ++w) mx = fmaxf(mx, part_ml[((w - 1) * GH + r) * 2]);
-        float den = 0.f;
-        float num[DI];
-        const float w0 = mx == -INFINITY ? 0.f : exp2f(m[r] - mx);
-        den = w0 * l[r];
+    for (int w = 0; w < NW - 1; ++w) mx = fmaxf(mx, part_ml[w][0][lane]);
+    const float w0 = mx == -INFINITY ? 0.f : exp2f(m - mx);
+    float den = w0 * l;
 #pragma unroll
-        for (int i = 0; i < DI; ++i) num[i] = w0 * acc[r][i];
-        for (int w = 1; w < NW; ++w) {
-            const float mw = part_ml[((w - 1) * GH + r) * 2];
-            const float ww = mx == -INFINITY ? 0.f : exp2f(mw - mx);
-            den += ww * part_ml[((w - 1) * GH + r) * 2 + 1];
-            const float* const pa = part_acc + ((w - 1) * GH + r) * D;
+    for (int e = 0; e < VE; ++e) acc[e] *= w0;
+    for (int w = 0; w < NW - 1; ++w) {
+        const float ww = mx == -INFINITY ? 0.f : exp2f(part_ml[w][0][lane] - mx);
+        den += ww * part_ml[w][1][lane];
+        if (ww == 0.f) continue;
 #pragma unroll
-            for (int i = 0; i < DI; ++i) {
-                const int d = lane + 64 * i;
-                if (d < D) num[i] += ww * pa[d];
-            }
-        }
-        if (a.splits > 1) {  // the split's partials, merged by general_merge
-            float* const po = a.part_o + part_index(r) * D;
+        for (int e = 0; e < VE; ++e)
 #pragma unroll
-            for (int i = 0; i < DI; ++i) {
-                const int d = lane + 64 * i;
-                if (d < D) po[d] = num[i];
-            }
-            if (lane == 0) {
-                a.part_ml[2 * part_index(r)] = mx;
-                a.part_ml[2 * part_index(r) + 1] = den;
-            }
-            continue;
-        }
-        const float inv = den > 0.f ? a.v_scale / den : 0.f;
-        T* const o = out + row_token(r) * a.ots + row_head(r) * a.ohs;
+            for (int v = 0; v < 4; ++v)
+                acc[e][v] += ww * part_acc[(w * VE * 4 + 4 * e + v) * 64 + lane];
+    }
+    float o[4 * VE];  // the lane's 4 * VE consecutive dims
 #pragma unroll
-        for (int i = 0; i < DI; ++i) {
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int e = 0; e < VE; ++e) o[v * VE + e] = acc[e][v];
+    const uint64_t bad = __ballot(col < nrows && !all_finite(o, den));
+    for (int r = 0; bad != 0 && r < nrows; ++r) {
+        if ((bad & (0x0001000100010001ull << r)) == 0) continue;
+        const int64_t tr = tok0 + r / hw;
+        const int hr = kvh * group + g0 + r % hw;
+        float em, el, eacc[(D + 63) / 64];
+        exact_row<T, F8, D>(a, static_cast<const T*>(a.q) + tr * a.qts + hr * a.qhs, kvh, table,
+                            k_begin, min(first_end + r / hw, k_end), em, el, eacc);
+        const int64_t pr = (item * a.heads + hr) * a.splits + split;
+#pragma unroll
+        for (int i = 0; i < (D + 63) / 64; ++i) {
             const int d = lane + 64 * i;
-            if (d < D) o[d] = static_cast<T>(num[i] * inv);
+            if (d >= D) continue;
+            if (a.splits > 1) a.part_o[pr * D + d] = eacc[i];
+            else out[tr * a.ots + hr * a.ohs + d] = static_cast<T>(eacc[i] * (a.v_scale / el));
+        }
+        if (a.splits > 1 && lane == 0) {
+            a.part_ml[2 * pr] = em;
+            a.part_ml[2 * pr + 1] = el;
+        }
+    }
+    if (col >= nrows || (bad >> col & 0x0001000100010001ull) != 0) return;
+    if (a.splits > 1) {  // the split's partials, merged by general_merge
+        float* const po = a.part_o + part * D + 4 * VE * quad;
+#pragma unroll
+        for (int i = 0; i < 4 * VE; i += 4)
+            *reinterpret_cast<float4*>(po + i) = make_float4(o[i], o[i + 1], o[i + 2], o[i + 3]);
+        if (quad == 0) {
+            a.part_ml[2 * part] = mx;
+            a.part_ml[2 * part + 1] = den;
+        }
+        return;
+    }
+    store_row<T>(out + token * a.ots + head * a.ohs + 4 * VE * quad, o,
+                 den > 0.f ? a.v_scale / den : 0.f, a.out_vec);
+}
+
+// Many query rows: prefill chunks. A workgroup of four waves serves up to
+// 64 * RT consecutive (query, head) rows of one KV head and item (row r is
+// query r / group, head r % group), 16 * RT per wave, each row with its own
+// causal bound. All waves walk the same keys, KC at a time, staged in LDS
+// for all of them: K as stored, V transposed into the k order of P.V, so
+// that every operand is one 16-byte LDS read. Two buffers, the next chunk's
+// global loads in flight while this one computes, one barrier per chunk.
+//
+// Bound by LDS bandwidth at RT = 1 (1 KiB of operand per 16-cycle MFMA and
+// wave, 4 waves against 128 bytes per cycle), which RT = 2 halves: taken when
+// its coarser tiles still give every CU a workgroup. In us, against the
+// vector-unit kernel: 4 x 512 queries over 2048 tokens, 32 query and 8 KV
+// heads of 64 2200 -> 121, of 256 6800 -> 352 (342 TFLOP/s); 2 x 256 over
+// 1033, 16 / 8 heads of 256 486 -> 61 (128 workgroups of one wave per SIMD).
+template <typename T, bool F8, int D, int RT>
+__global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(GeneralAttention a) {
+    constexpr int KC = D > 128 ? 32 : 64;  // keys per chunk
+    constexpr int KS = D / 32;             // Q.K^T steps
+    constexpr int DT = D / 16;             // 16-dim tiles of the output
+    constexpr int G = KC / 32;             // P.V steps
+    constexpr int NT = 64 * kRowWaves;
+    // Row strides padded by 16 bytes: the 16 rows that a quarter wave reads
+    // at once start 4 banks apart.
+    constexpr int KSTR = D * 2 + 16, VSTR = KC * 2 + 16;
+    constexpr int kBuf = KC * KSTR + D * VSTR;
+    __shared__ __align__(16) unsigned char smem[2 * kBuf];
+    __shared__ int64_t row_off[2][KC];  // byte offsets of a chunk's cache rows
+    const int wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int col = lane & 15, quad = lane >> 4;
+
+    const int group = a.heads / a.kv_heads;
+    const int kvh = int(blockIdx.x % a.kv_heads);
+    const int64_t item = blockIdx.x / a.kv_heads;
+    const int64_t tok0 = a.q_offsets[item];
+    const int64_t qlen = a.q_offsets[item + 1] - tok0;
+    const int64_t total = qlen * group;
+    const int64_t r0 = int64_t(blockIdx.y) * (64 * RT);
+    if (r0 >= total) return;  // uniform per workgroup
+    const int64_t ctx = a.lengths[item];
+    const int64_t before = ctx - qlen;
+    const int64_t last = min(r0 + 64 * RT, total) - 1;  // the workgroup's last row
+    const int64_t kv_max = before + last / group + 1;   // and the keys it sees
+    T* const out = static_cast<T*>(a.out);
+    const int64_t wr0 = r0 + wave * 16 * RT;  // the wave's first row
+
+    U16x8 qb[RT][KS];
+    int64_t bound[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int64_t r = wr0 + 16 * t + col;
+        const bool has = r < total;
+        const int64_t query = (has ? r : 0) / group;
+        const int head = kvh * group + int((has ? r : 0) % group);
+        bound[t] = has ? before + query + 1 : 0;
+        const T* const q = static_cast<const T*>(a.q) + (tok0 + query) * a.qts + head * a.qhs +
+                           8 * quad;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            qb[t][s] = load_query<T>(q + 32 * s, a.q_vec);
+            if (!has) qb[t][s] = U16x8{};
+        }
+    }
+    // Keys beyond the wave's last row's bound are none of its business.
+    const int64_t wave_end = wr0 < total
+        ? before + min(wr0 + 16 * RT - 1, total - 1) / group + 1 : 0;
+    const float qscale = a.scale * kLog2eG * a.k_scale;
+
+    gf32x4 acc[RT][DT];  // acc[t][d][v]: dim 16 * d + 4 * quad + v of row 16 * t + col
+    float m[RT], l[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        m[t] = -INFINITY;
+        l[t] = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) acc[t][d] = gf32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // Staging. K: 8-element pieces, a key's pieces side by side in the lanes.
+    // V: 4 keys x 8 dims per task, transposed in registers; 8 lanes hold 64
+    // dims of the same keys (one 128-byte line each), 8 groups of lanes the
+    // keys of a 32-key step.
+    constexpr int kPieces = KC * (D / 8);
+    constexpr int kPer = (kPieces + NT - 1) / NT;
+    constexpr int kTasks = (KC / 4) * (D / 8);
+    constexpr int kVPer = (kTasks + NT - 1) / NT;
+    using Piece = std::conditional_t<F8, uint2, U16x8>;
+    constexpr int EB = F8 ? 1 : 2;
+    Piece kst[kPer], vst[kVPer][4];
+    const int64_t table = a.offsets[item];
+    const uint32_t bs = uint32_t(a.block_size);
+    const char* const kc = static_cast<const char*>(a.k) + int64_t(kvh) * a.chs * EB;
+    const char* const vc = static_cast<const char*>(a.v) + int64_t(kvh) * a.chs * EB;
+    // Thread x < KC resolves key x of each chunk (past the end: the last key, a
+    // valid row): its block id two chunks ahead of the chunk's loads, its
+    // byte offset into LDS one chunk ahead, for all threads.
+    auto load_id = [&](int64_t t0) -> int64_t {
+        return a.blocks[table + uint32_t(min(t0 + int(threadIdx.x) % KC, kv_max - 1)) / bs];
+    };
+    auto put_offset = [&](int64_t t0, int64_t id, int slot) {
+        const uint32_t t = uint32_t(min(t0 + int(threadIdx.x) % KC, kv_max - 1));
+        if (threadIdx.x < KC) row_off[slot][threadIdx.x] = (id * bs + t % bs) * a.css * EB;
+    };
+    // Task x: 8-dim piece `oct` of keys 4 * kq .. + 3.
+    auto v_task = [&](int x, int& oct, int& kq) {
+        constexpr int OW = D / 8 < 8 ? D / 8 : 8;  // pieces side by side in the lanes
+        const int inner = x % (OW * (KC / 4));
+        oct = x / (OW * (KC / 4)) * OW + inner % OW;
+        kq = inner / OW;
+    };
+    auto load_stage = [&](int slot) {
+        const int64_t* const ro = row_off[slot];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int x = int(threadIdx.x) + u * NT;
+            if (kPieces % NT != 0 && x >= kPieces) break;
+            kst[u] = *reinterpret_cast<const Piece*>(kc + ro[x / (D / 8)] +
+                                                     (x % (D / 8)) * 8 * EB);
+        }
+#pragma unroll
+        for (int u = 0; u < kVPer; ++u) {
+            const int x = int(threadIdx.x) + u * NT;
+            if (kTasks % NT != 0 && x >= kTasks) break;
+            int oct, kq;
+            v_task(x, oct, kq);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                vst[u][i] = *reinterpret_cast<const Piece*>(vc + ro[4 * kq + i] +
+                                                            oct * 8 * EB);
+        }
+    };
+    auto widen = [&](const Piece& x) -> U16x8 {
+        if constexpr (F8) return fp8x8_widen<T>(x);
+        else return x;
+    };
+    auto store_stage = [&](unsigned char* buf) {
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int x = int(threadIdx.x) + u * NT;
+            if (kPieces % NT != 0 && x >= kPieces) break;
+            *reinterpret_cast<U16x8*>(buf + (x / (D / 8)) * KSTR + (x % (D / 8)) * 16) =
+                widen(kst[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kVPer; ++u) {
+            const int x = int(threadIdx.x) + u * NT;
+            if (kTasks % NT != 0 && x >= kTasks) break;
+            int oct, kq;
+            v_task(x, oct, kq);
+            const U16x8 r0v = widen(vst[u][0]), r1v = widen(vst[u][1]);
+            const U16x8 r2v = widen(vst[u][2]), r3v = widen(vst[u][3]);
+            // Keys 4 * kq .. + 3 of 32-key group kq / 8: tile (kq % 8) / 4,
+            // quad kq % 4, so k = 8 * quad + 4 * tile + i.
+            const int pos = 32 * (kq / 8) + 8 * (kq & 3) + 4 * ((kq & 7) >> 2);
+            unsigned char* const vt = buf + KC * KSTR + oct * 8 * VSTR + pos * 2;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                *reinterpret_cast<uint2*>(vt + (2 * w) * VSTR) =
+                    make_uint2(pair_lo(r0v.w[w], r1v.w[w]), pair_lo(r2v.w[w], r3v.w[w]));
+                *reinterpret_cast<uint2*>(vt + (2 * w + 1) * VSTR) =
+                    make_uint2(pair_hi(r0v.w[w], r1v.w[w]), pair_hi(r2v.w[w], r3v.w[w]));
+            }
+        }
+    };
+
+    int64_t id = 0;
+    if (kv_max > 0) {  // uniform per workgroup
+        put_offset(0, load_id(0), 0);
+        id = load_id(KC);
+        __syncthreads();
+        load_stage(0);
+    }
+    asm volatile("" ::: "memory");  // keeps carried loads where they are issued
+    int cur = 0;
+    for (int64_t t0 = 0; t0 < kv_max; t0 += KC, cur ^= 1) {
+        unsigned char* const buf = smem + cur * kBuf;
+        store_stage(buf);
+        put_offset(t0 + KC, id, cur ^ 1);
+        // After it, every wave is also past the reads of what the next
+        // iteration overwrites (the other buffer, these offsets' predecessors).
+        __syncthreads();
+        id = load_id(t0 + 2 * KC);
+        load_stage(cur ^ 1);
+        if (t0 >= wave_end) continue;
+        const unsigned char* const ks = buf + col * KSTR + quad * 16;
+        const unsigned char* const vs = buf + KC * KSTR + col * VSTR + quad * 16;
+        // Operands are read ahead of the MFMAs that take them, all of K's at
+        // once and V's behind Q.K^T: the compiler's own order reads one or two
+        // ahead and waits out the LDS latency 32 times per chunk.
+        U16x8 kk[2 * G][KS];
+#pragma unroll
+        for (int j = 0; j < 2 * G; ++j)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+                kk[j][s] = *reinterpret_cast<const U16x8*>(ks + 16 * j * KSTR + 64 * s);
+        __builtin_amdgcn_sched_barrier(0);
+        gf32x4 sc[RT][2 * G];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2 * G; ++j) sc[t][j] = gf32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 2 * G; ++j)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int t = 0; t < RT; ++t) sc[t][j] = mfma32<T>(kk[j][s], qb[t][s], sc[t][j]);
+        U16x8 vv[DT][G];
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                vv[d][g] = *reinterpret_cast<const U16x8*>(vs + 16 * d * VSTR + 64 * g);
+        __builtin_amdgcn_sched_barrier(0);
+        U16x8 hi[RT][G], lo[RT][G];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            float x[8 * G];
+            const int left = int(max<int64_t>(min<int64_t>(bound[t] - t0, KC), 0)) - 4 * quad;
+#pragma unroll
+            for (int j = 0; j < 2 * G; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    x[4 * j + i] = 16 * j + i < left ? sc[t][j][i] * qscale : -INFINITY;
+            float alpha;
+            if (softmax_step(x, m[t], l[t], alpha)) {
+#pragma unroll
+                for (int d = 0; d < DT; ++d) acc[t][d] *= alpha;
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[i] = x[8 * g + i];
+                split_p<T>(p, hi[t][g], lo[t][g]);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int t = 0; t < RT; ++t) {
+                    acc[t][d] = mfma32<T>(vv[d][g], hi[t][g], acc[t][d]);
+                    acc[t][d] = mfma32<T>(vv[d][g], lo[t][g], acc[t][d]);
+                }
+    }
+
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const float den = quad_sum(l[t]);
+        const float inv = den > 0.f ? a.v_scale / den : 0.f;
+        const int64_t r = wr0 + 16 * t + col;
+        bool ok = den < INFINITY;  // false for NaN too
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) ok = ok && fabsf(acc[t][d][v]) < INFINITY;
+        const uint64_t bad = __ballot(r < total && !ok);
+        for (int c = 0; bad != 0 && c < 16; ++c) {
+            if ((bad & (0x0001000100010001ull << c)) == 0) continue;
+            const int64_t rc = wr0 + 16 * t + c, qc = rc / group;
+            const int hc = kvh * group + int(rc % group);
+            float em, el, eacc[(D + 63) / 64];
+            exact_row<T, F8, D>(a, static_cast<const T*>(a.q) + (tok0 + qc) * a.qts + hc * a.qhs,
+                                kvh, table, 0, before + qc + 1, em, el, eacc);
+#pragma unroll
+            for (int i = 0; i < (D + 63) / 64; ++i) {
+                const int d = lane + 64 * i;
+                if (d < D)
+                    out[(tok0 + qc) * a.ots + hc * a.ohs + d] =
+                        static_cast<T>(eacc[i] * (a.v_scale / el));
+            }
+        }
+        if (r >= total || (bad >> col & 0x0001000100010001ull) != 0) continue;
+        T* const o = out + (tok0 + r / group) * a.ots +
+                     (kvh * group + int(r % group)) * a.ohs + 4 * quad;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            const float x[4] = {acc[t][d][0], acc[t][d][1], acc[t][d][2], acc[t][d][3]};
+            store_row<T>(o + 16 * d, x, inv, a.out_vec);
         }
     }
 }
@@ -611,6 +1096,12 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     const bool rows_kernel = vec && rows_kernel_dim(D);
     const int group = g.heads / g.kv_heads;
     const int64_t qpw = rows_kernel && group < GH ? GH / group : 1;
+    g.q_vec = g.qts % 8 == 0 && g.qhs % 8 == 0 && aligned16(g.q);
+    g.out_vec = g.ots % 4 == 0 && g.ohs % 4 == 0 && aligned8(g.out);
+    // Prefill (head dim 128 has its own kernel): the tiled kernel from 32 rows per item and KV head (where two
+    // of its waves have rows); below, four waves share the keys of 16 rows.
+    const int64_t item_rows = g.max_query_len * group;
+    const bool tiles = rows_kernel && D != 128 && !g.rows && item_rows > 2 * GH;
     g.splits = 1;
     g.split_keys = 0;
     g.part_o = g.part_ml = nullptr;
@@ -635,10 +1126,29 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
                     1u};
     return dispatch_half(g.dtype, [&]<int DT>() {
         using T = typename Elem<DT>::T;
-        if (rows_kernel) {
+        if (tiles) {
+            // 128 rows per workgroup where that leaves one for every CU.
+            const int64_t units = g.num_items * g.kv_heads;
+            const bool wide = units * ((item_rows + 127) / 128) >= 256;
+            const int64_t ty = (item_rows + (wide ? 127 : 63)) / (wide ? 128 : 64);
+            TVLLM_CHECK(units <= INT32_MAX && ty <= 65535, "attention: launch grid out of range");
+            const dim3 tg{static_cast<uint32_t>(units), static_cast<uint32_t>(ty), 1u};
+            auto go = [&]<int DD, int RT>() {
+                if (f8) tiles_attention_kernel<T, true, DD, RT><<<tg, 64 * kRowWaves, 0, stream>>>(g);
+                else tiles_attention_kernel<T, false, DD, RT><<<tg, 64 * kRowWaves, 0, stream>>>(g);
+            };
+            auto rt = [&]<int DD>() {
+                if (wide) go.template operator()<DD, 2>();
+                else go.template operator()<DD, 1>();
+            };
+            if (D == 32) rt.template operator()<32>();
+            else if (D == 64) rt.template operator()<64>();
+            else rt.template operator()<256>();
+        } else if (rows_kernel) {
             auto go = [&]<int DD>() {
-                if (f8) rows_attention_kernel<T, true, DD><<<grid, 64 * kRowWaves, 0, stream>>>(g);
-                else rows_attention_kernel<T, false, DD><<<grid, 64 * kRowWaves, 0, stream>>>(g);
+                constexpr int threads = 64 * kRowWaves;
+                if (f8) rows_attention_kernel<T, true, DD><<<grid, threads, 0, stream>>>(g);
+                else rows_attention_kernel<T, false, DD><<<grid, threads, 0, stream>>>(g);
             };
             if (D == 32) go.template operator()<32>();
             else if (D == 64) go.template operator()<64>();
