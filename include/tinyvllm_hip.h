@@ -250,6 +250,22 @@ int tvllm_paged_decode_qk_norm_rope_partials(
     void* workspace, int64_t workspace_bytes, int dtype, int cache_dtype, float k_scale,
     float v_scale, tvllm_stream_t stream);
 
+/* y = x @ weight^T for up to 64 rows x [rows, width] (element row stride, last
+ * stride 1) and a dense weight [columns, width], accumulated in fp32:
+ *   silu == 0, slices == 0: out [rows, columns] of dtype, rounded once;
+ *   slices > 0: out float [slices, rows, columns], the partial products over
+ *     that many consecutive parts of the width (what
+ *     tvllm_add_rms_norm_partials takes);
+ *   silu != 0: weight packs [gate | up] rows; out [rows, columns / 2] is
+ *     tvllm_silu_and_mul of the rounded projection.
+ * width and columns multiples of 32; x, weight and out 16-byte aligned.
+ * Replaces: F.linear of a decode step's small projections (reference
+ *           tinyvllm/layers.py:80-125), and with silu the silu_and_mul
+ *           behind it (reference tinyvllm/kernels/pointwise.cu:619-680). */
+int tvllm_few_rows_linear(const void* x, int64_t x_row_stride, const void* weight,
+                          int64_t rows, int64_t columns, int64_t width, void* out,
+                          int64_t slices, int silu, int dtype, tvllm_stream_t stream);
+
 /* RMSNorm over rows of width `width`, optionally after a residual add:
  *   x = residual ? round(x + residual) : x
  *   out = round(round(x * rsqrt(mean(x^2) + eps)) * weight)

@@ -1,7 +1,9 @@
 """Qwen3 building blocks (reference: tinyvllm/layers.py:19-251).
 
-Dense projections stay on PyTorch-ROCm GEMMs (hipBLASLt); normalisation and
-activation run on the HIP kernels of ``tinyvllm.kernels.pointwise``.
+Dense projections run on PyTorch-ROCm GEMMs (hipBLASLt), except the small ones
+of a decode batch, which those leave most of the GPU idle for
+(``tinyvllm.kernels.linear``); normalisation and activation run on the HIP
+kernels of ``tinyvllm.kernels.pointwise``.
 """
 from __future__ import annotations
 
@@ -13,6 +15,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from tinyvllm._validation import _check_positive_int
+from tinyvllm.kernels import linear as few_rows
 from tinyvllm.kernels.pointwise import (
     add_rms_norm, add_rms_norm_partials, rms_norm, silu_and_mul,
 )
@@ -57,7 +60,36 @@ class PackedLinear(nn.Module):
         self.reset_parameters()
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if self.takes_few_rows(x):
+            return few_rows.few_rows_linear(x, self.weight)
         return F.linear(x, self.weight)
+
+    def takes_few_rows(self, x: torch.Tensor) -> bool:
+        """Whether this call runs on the few-rows kernel: up to 64 rows with a
+        weight of at most 2^22 elements, up to 32 with 2^23. Measured on
+        MI355X (bf16, cold weights, us, F.linear -> kernel): 1024 -> 4096
+        (2^22) 16 rows 7.6 -> 4.6, 64 rows 11.6 -> 7.4; 2048 -> 4096 (2^23)
+        16 rows 11.7 -> 6.7, 32 rows 11.9 -> 8.3, 64 rows 12.4 -> 12.1; 4096
+        -> 6144 16 rows 14.4 -> 15.7, 64 rows 17.8 -> 25.7."""
+        limit = 1 << (22 if x.dim() == 2 and x.shape[0] > 32 else 23)
+        return self.weight.numel() <= limit and few_rows.fits(x, self.weight)
+
+    def gated(self, x: torch.Tensor) -> torch.Tensor | None:
+        """silu(gate) * up of a [gate | up] projection in one launch, or None
+        where the projection and the activation on their own are faster: up
+        to 16 rows with weights of at most 2^27 elements, up to 64 with 2^23.
+        Measured on MI355X (bf16, cold weights, us, F.linear + silu_and_mul
+        -> kernel): 1024 -> 6144 16 / 64 rows 10.9 / 14.7 -> 6.3 / 8.9; 2048
+        -> 12288 16 rows 18.1 -> 16.1, 32 rows 18.1 -> 19.5; 4096 -> 24576 1
+        / 16 rows 47.2 / 46.1 -> 37.2 / 44.4, 64 rows 50.9 -> 73; 5120 ->
+        51200 1 row 91.7 -> 127."""
+        if len(self.output_sizes) != 2 or self.output_sizes[0] != self.output_sizes[1]:
+            return None
+        limit = 1 << (23 if x.dim() == 2 and x.shape[0] > 16 else 27)
+        if (self.weight.numel() > limit or self.output_sizes[0] % 16
+                or not few_rows.fits(x, self.weight)):
+            return None
+        return few_rows.few_rows_linear(x, self.weight, silu=True)
 
     def decode_partials(self, x: torch.Tensor, splits: int = 4) -> torch.Tensor | None:
         """fp32 [splits, rows, out] partial products over ``splits`` slices of
@@ -160,6 +192,19 @@ class SplitKLinear(nn.Linear):
         return s if self.in_features % (8 * s) == 0 else 1
 
     def forward(self, x: torch.Tensor) -> torch.Tensor | SplitKPartials:
+        # Narrow outputs of a decode batch: the same slices on the few-rows
+        # kernel, up to 64 rows with weights of at most 2^22 elements, up to
+        # 32 with 13 M. Measured on MI355X (eight slices, us, bmm -> kernel):
+        # 2048 -> 1024 16 / 64 rows 6.0 / 5.9 -> 3.5 / 5.0; 3072 -> 1024 8.0 /
+        # 7.9 -> 4.1 / 6.0; 2048 -> 2048 7.0 / 7.2 -> 4.5 / 6.5; 6144 -> 2048
+        # 16 rows 8.9 -> 8.7, 64 rows 11.6 -> 12.8.
+        if (self.out_features <= 2048 and x.dim() == 2
+                and self.weight.numel() <= (1 << 22 if x.shape[0] > 32 else 13 << 20)
+                and few_rows.fits(x, self.weight)):
+            s = self.splits_for(x.shape[0])
+            if s > 1:
+                return SplitKPartials(
+                    few_rows.few_rows_linear(x, self.weight, slices=s), x.dtype)
         # Split-K views the rows in place: only for contiguous 2-D GPU inputs
         # (torch.bmm with an fp32 out_dtype is a GPU-only overload).
         split_ok = x.dim() == 2 and x.is_cuda and x.is_contiguous()

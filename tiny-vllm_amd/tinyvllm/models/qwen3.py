@@ -3,7 +3,8 @@
 Per layer (reference op order, qwen3.py:263-303 and :386-412):
   add_rms_norm -> qkv GEMM -> QK-norm + RoPE (+ KV write) -> paged attention
   -> o GEMM -> add_rms_norm -> gate_up GEMM -> SiLU*up -> down GEMM.
-GEMMs are PyTorch-ROCm ``F.linear``; everything else is a HIP kernel. When the
+GEMMs are PyTorch-ROCm ``F.linear`` (small decode projections: the few-rows
+kernel, with the SiLU in its epilogue); everything else is a HIP kernel. When the
 attention backend offers ``prepare_qkv`` (the native backend does), the
 QK-norm/RoPE kernel also writes K/V into the paged cache, so the separate
 store_kv launch of the reference disappears.
@@ -155,7 +156,8 @@ class Qwen3Attention(nn.Module):
         # Decode-only steps on a backend that takes the qkv projection as
         # split-K partials: the fused decode kernel sums them itself.
         from_partials = getattr(attention, "attend_qkv_partials", None)
-        if from_partials is not None and attention.takes_qkv_partials(self.num_heads):
+        if (from_partials is not None and attention.takes_qkv_partials(self.num_heads)
+                and not self.qkv_proj.takes_few_rows(hidden_states)):
             parts = self.qkv_proj.decode_partials(hidden_states)
             if parts is not None:
                 out = from_partials(layer_idx, parts, self.num_heads, self.q_norm.weight,
@@ -191,7 +193,13 @@ class Qwen3MLP(nn.Module):
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor | SplitKPartials:
         """Returns SplitKPartials for decode-sized batches (consumed by the
         next RMSNorm.add)."""
-        return self.down_proj(self.act_fn(self.gate_up_proj(hidden_states)))
+        gated = None
+        if not any(m._forward_hooks or m._forward_pre_hooks
+                   for m in (self.gate_up_proj, self.act_fn)):  # only their own calls serve hooks
+            gated = self.gate_up_proj.gated(hidden_states)
+        if gated is None:
+            gated = self.act_fn(self.gate_up_proj(hidden_states))
+        return self.down_proj(gated)
 
 
 class Qwen3DecoderLayer(nn.Module):
