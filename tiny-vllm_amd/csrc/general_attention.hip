@@ -717,15 +717,19 @@ rows_attention_kernel(GeneralAttention a) {
 // for all of them: K as stored, V transposed into the k order of P.V, so
 // that every operand is one 16-byte LDS read. Two buffers, the next chunk's
 // global loads in flight while this one computes, one barrier per chunk.
+// With HV = 2 a second set of four waves takes every other chunk of the same
+// rows' keys through buffers of its own, and the two merge at the end.
 //
-// Bound by LDS bandwidth at RT = 1 (1 KiB of operand per 16-cycle MFMA and
-// wave, 4 waves against 128 bytes per cycle), which RT = 2 halves: taken when
-// its coarser tiles still give every CU a workgroup. In us, against the
-// vector-unit kernel: 4 x 512 queries over 2048 tokens, 32 query and 8 KV
-// heads of 64 2200 -> 121, of 256 6800 -> 352 (342 TFLOP/s); 2 x 256 over
-// 1033, 16 / 8 heads of 256 486 -> 61 (128 workgroups of one wave per SIMD).
-template <typename T, bool F8, int D, int RT>
-__global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(GeneralAttention a) {
+// Bound by the instruction stream of a SIMD's waves (softmax and staging
+// against 48 MFMAs per 32 keys at head dim 256) and by LDS bandwidth at RT = 1
+// (1 KiB of operand per 16-cycle MFMA and wave). Registers are held to 256, so
+// that two waves share a SIMD. In us, against the vector-unit kernel: 4 x 512
+// queries over 2048 tokens, 32 query and 8 KV heads of 64 2257 -> 84 (357
+// TFLOP/s), of 256 6566 -> 329 (366 TFLOP/s); 2 x 256 over 1033, 16 / 8 heads
+// of 256 488 -> 53.
+template <typename T, bool F8, int D, int RT, int HV>
+__global__ void __launch_bounds__(64 * kRowWaves * HV, 2)
+tiles_attention_kernel(GeneralAttention a) {
     constexpr int KC = D > 128 ? 32 : 64;  // keys per chunk
     constexpr int KS = D / 32;             // Q.K^T steps
     constexpr int DT = D / 16;             // 16-dim tiles of the output
@@ -735,10 +739,14 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
     // at once start 4 banks apart.
     constexpr int KSTR = D * 2 + 16, VSTR = KC * 2 + 16;
     constexpr int kBuf = KC * KSTR + D * VSTR;
-    __shared__ __align__(16) unsigned char smem[2 * kBuf];
-    __shared__ int64_t row_off[2][KC];  // byte offsets of a chunk's cache rows
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
+    __shared__ __align__(16) unsigned char smem_all[HV * 2 * kBuf];
+    __shared__ int64_t row_offs[HV][2][KC];  // byte offsets of a chunk's cache rows
+    const int half = HV == 1 ? 0 : threadIdx.x / NT;
+    const int tid = threadIdx.x % NT;  // within the half
+    unsigned char* const smem = smem_all + half * 2 * kBuf;
+    int64_t (*const row_off)[KC] = row_offs[half];
+    const int wave = tid >> 6;
+    const int lane = tid & 63;
     const int col = lane & 15, quad = lane >> 4;
 
     const int group = a.heads / a.kv_heads;
@@ -807,11 +815,11 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
     // valid row): its block id two chunks ahead of the chunk's loads, its
     // byte offset into LDS one chunk ahead, for all threads.
     auto load_id = [&](int64_t t0) -> int64_t {
-        return a.blocks[table + uint32_t(min(t0 + int(threadIdx.x) % KC, kv_max - 1)) / bs];
+        return a.blocks[table + uint32_t(min(t0 + tid % KC, kv_max - 1)) / bs];
     };
     auto put_offset = [&](int64_t t0, int64_t id, int slot) {
-        const uint32_t t = uint32_t(min(t0 + int(threadIdx.x) % KC, kv_max - 1));
-        if (threadIdx.x < KC) row_off[slot][threadIdx.x] = (id * bs + t % bs) * a.css * EB;
+        const uint32_t t = uint32_t(min(t0 + tid % KC, kv_max - 1));
+        if (tid < KC) row_off[slot][tid] = (id * bs + t % bs) * a.css * EB;
     };
     // Task x: 8-dim piece `oct` of keys 4 * kq .. + 3.
     auto v_task = [&](int x, int& oct, int& kq) {
@@ -824,14 +832,14 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
         const int64_t* const ro = row_off[slot];
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int x = int(threadIdx.x) + u * NT;
+            const int x = tid + u * NT;
             if (kPieces % NT != 0 && x >= kPieces) break;
             kst[u] = *reinterpret_cast<const Piece*>(kc + ro[x / (D / 8)] +
                                                      (x % (D / 8)) * 8 * EB);
         }
 #pragma unroll
         for (int u = 0; u < kVPer; ++u) {
-            const int x = int(threadIdx.x) + u * NT;
+            const int x = tid + u * NT;
             if (kTasks % NT != 0 && x >= kTasks) break;
             int oct, kq;
             v_task(x, oct, kq);
@@ -848,14 +856,14 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
     auto store_stage = [&](unsigned char* buf) {
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int x = int(threadIdx.x) + u * NT;
+            const int x = tid + u * NT;
             if (kPieces % NT != 0 && x >= kPieces) break;
             *reinterpret_cast<U16x8*>(buf + (x / (D / 8)) * KSTR + (x % (D / 8)) * 16) =
                 widen(kst[u]);
         }
 #pragma unroll
         for (int u = 0; u < kVPer; ++u) {
-            const int x = int(threadIdx.x) + u * NT;
+            const int x = tid + u * NT;
             if (kTasks % NT != 0 && x >= kTasks) break;
             int oct, kq;
             v_task(x, oct, kq);
@@ -876,22 +884,25 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
     };
 
     int64_t id = 0;
+    constexpr int kStep = HV * KC;
+    const int64_t first = half * KC;
     if (kv_max > 0) {  // uniform per workgroup
-        put_offset(0, load_id(0), 0);
-        id = load_id(KC);
+        put_offset(first, load_id(first), 0);
+        id = load_id(first + kStep);
         __syncthreads();
         load_stage(0);
     }
     asm volatile("" ::: "memory");  // keeps carried loads where they are issued
     int cur = 0;
-    for (int64_t t0 = 0; t0 < kv_max; t0 += KC, cur ^= 1) {
+    for (int64_t step = 0; step < kv_max; step += kStep, cur ^= 1) {
+        const int64_t t0 = step + first;  // this half's chunk
         unsigned char* const buf = smem + cur * kBuf;
         store_stage(buf);
-        put_offset(t0 + KC, id, cur ^ 1);
+        put_offset(t0 + kStep, id, cur ^ 1);
         // After it, every wave is also past the reads of what the next
         // iteration overwrites (the other buffer, these offsets' predecessors).
         __syncthreads();
-        id = load_id(t0 + 2 * KC);
+        id = load_id(t0 + 2 * kStep);
         load_stage(cur ^ 1);
         if (t0 >= wave_end) continue;
         const unsigned char* const ks = buf + col * KSTR + quad * 16;
@@ -958,6 +969,41 @@ __global__ void __launch_bounds__(64 * kRowWaves) tiles_attention_kernel(General
                 }
     }
 
+    if constexpr (HV > 1) {
+        // The second half's (max, sum, accumulators) join the first's, lane by
+        // lane, through the staging buffers.
+        __syncthreads();  // every wave is past its reads of them
+        float* const part = reinterpret_cast<float*>(smem_all) + wave * 64 + lane;
+        constexpr int kStride = 64 * kRowWaves;
+        static_assert((RT * (4 * DT + 2)) * kStride * 4 <= HV * 2 * kBuf, "merge fits the buffers");
+        if (half == 1) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                float* const p = part + t * (4 * DT + 2) * kStride;
+                p[0] = m[t];
+                p[kStride] = l[t];
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) p[(2 + 4 * d + v) * kStride] = acc[t][d][v];
+            }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const float* const p = part + t * (4 * DT + 2) * kStride;
+            const float mx = fmaxf(m[t], p[0]);
+            const float w0 = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[t] - mx);
+            const float w1 = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(p[0] - mx);
+            l[t] = w0 * l[t] + w1 * p[kStride];
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    acc[t][d][v] = w0 * acc[t][d][v] + w1 * p[(2 + 4 * d + v) * kStride];
+        }
+    }
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
         const float den = quad_sum(l[t]);
@@ -1127,19 +1173,34 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     return dispatch_half(g.dtype, [&]<int DT>() {
         using T = typename Elem<DT>::T;
         if (tiles) {
-            // 128 rows per workgroup where that leaves one for every CU.
+            // 128 rows per workgroup where that leaves one for every CU (4 x
+            // 512 queries over 2048 tokens, 32 / 8 heads of 64: 84 us against
+            // 99 with 64 rows; heads of 256 gain nothing, 320 against 329, and
+            // lose where tiles are few, 72 against 63 us for 3 x 300). Where
+            // 64 rows do not fill the CUs either, two halves of a workgroup
+            // share the keys (2 x 256 over 1033, heads of 256: 61 -> 53 us; 8
+            // x 40 over 2040, FP8, heads of 64: 43 -> 35 us); at full grids
+            // the halves only add their merge (99 -> 112 us).
             const int64_t units = g.num_items * g.kv_heads;
-            const bool wide = units * ((item_rows + 127) / 128) >= 256;
+            const bool wide = D <= 64 && units * ((item_rows + 127) / 128) >= 256;
             const int64_t ty = (item_rows + (wide ? 127 : 63)) / (wide ? 128 : 64);
+            const bool halves = units * ty < 256;
             TVLLM_CHECK(units <= INT32_MAX && ty <= 65535, "attention: launch grid out of range");
             const dim3 tg{static_cast<uint32_t>(units), static_cast<uint32_t>(ty), 1u};
-            auto go = [&]<int DD, int RT>() {
-                if (f8) tiles_attention_kernel<T, true, DD, RT><<<tg, 64 * kRowWaves, 0, stream>>>(g);
-                else tiles_attention_kernel<T, false, DD, RT><<<tg, 64 * kRowWaves, 0, stream>>>(g);
+            auto go = [&]<int DD, int RT, int HV>() {
+                constexpr int threads = 64 * kRowWaves * HV;
+                if (f8) tiles_attention_kernel<T, true, DD, RT, HV><<<tg, threads, 0, stream>>>(g);
+                else tiles_attention_kernel<T, false, DD, RT, HV><<<tg, threads, 0, stream>>>(g);
             };
             auto rt = [&]<int DD>() {
-                if (wide) go.template operator()<DD, 2>();
-                else go.template operator()<DD, 1>();
+                if constexpr (DD <= 64) {
+                    if (wide) {
+                        go.template operator()<DD, 2, 1>();
+                        return;
+                    }
+                }
+                if (halves) go.template operator()<DD, 1, 2>();
+                else go.template operator()<DD, 1, 1>();
             };
             if (D == 32) rt.template operator()<32>();
             else if (D == 64) rt.template operator()<64>();
