@@ -395,12 +395,10 @@ int tvllm_resolve_tokens(int64_t* tokens, const int64_t* src, const int64_t* pre
  * general kernel of tvllm_paged_decode (fp32; a workgroup per KV head and
  * up to 16 (query token, query head) rows of one item).
  * workspace: >= tvllm_paged_prefill_workspace_size(dtype, cache_dtype)
- * bytes, 4-byte aligned, zero before the first call; every call leaves it
- * zero. (A bf16 cache's V is converted to fp16 for the P.V products; a call
- * in which a V value of 65536 or more in magnitude, an infinity or a NaN
- * enters a product raises a flag there, and a second, exact launch
- * recomputes it. Calls that share one workspace must be ordered on one
- * stream.)
+ * bytes, 4-byte aligned; left as it is. (A bf16 cache's V is converted to
+ * fp16 for the P.V products; a workgroup in which a V value of 65536 or more
+ * in magnitude, an infinity or a NaN enters a product redoes its queries
+ * exactly. The flag that once asked for that lived in the workspace.)
  * Replaces: CudaAttention._attend's per-row gather + SDPA for rows with
  * history (reference tinyvllm/runtime/attention.py:102-151, 235-285). */
 int tvllm_paged_prefill(const void* q, int64_t q_token_stride,
@@ -418,8 +416,8 @@ int tvllm_paged_prefill(const void* q, int64_t q_token_stride,
                         int dtype, int cache_dtype, float k_scale,
                         float v_scale, tvllm_stream_t stream);
 
-/* Bytes of workspace tvllm_paged_prefill needs: 8 for a bf16 query and
- * cache (the fallback guard), 0 otherwise. No counterpart in the reference
+/* Bytes of workspace tvllm_paged_prefill asks for: 8 for a bf16 query and
+ * cache, 0 otherwise. No counterpart in the reference
  * (its prefill path allocates nothing of the kind). */
 int64_t tvllm_paged_prefill_workspace_size(int dtype, int cache_dtype);
 

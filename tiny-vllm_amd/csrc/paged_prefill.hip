@@ -27,10 +27,10 @@
 //    output, the whole bf16 tolerance), and a bf16 cache's V is converted to
 //    fp16 as it is staged, which is exact below 65536. A V value beyond that
 //    (or an infinity or NaN) becomes an fp16 infinity or NaN and makes the
-//    outputs it reaches non-finite; a wave whose accumulators end
-//    non-finite raises a guard, and a second launch recomputes the call on
-//    bf16 MFMAs with P as a rounded value plus its rounded remainder (about
-//    16 bits of P, two MFMAs per product).
+//    outputs it reaches non-finite; a workgroup with a wave whose
+//    accumulators end so recomputes its queries on bf16 MFMAs with P as a
+//    rounded value plus its rounded remainder (about 16 bits of P, two MFMAs
+//    per product).
 //    The O^T accumulator of a lane belongs to its own query: the softmax
 //    rescale and the final 1/l are lane-local.
 //  * online softmax in base 2 (v_exp_f32) with one running (max, sum) per
@@ -87,9 +87,6 @@ __device__ __forceinline__ int vt_pos(int tq) {
 // tiles skip the rescale of the output accumulators.
 constexpr float kSlack = 8.f;
 
-// Workgroups of the exact fallback launch (each loops over tasks).
-constexpr int64_t kExactWorkgroups = 32;
-
 template <typename T>
 struct PrefillArgs {
     const T* q;
@@ -106,7 +103,6 @@ struct PrefillArgs {
     int heads, kv_heads, block_size, block_shift, q_tiles, grid;
     float scale_log2;  // softmax scale * log2(e) (* k_scale for an FP8 cache)
     float v_scale;     // FP8 cache: V dequantisation scale (1 otherwise)
-    int* guard;        // bf16 cache: [recompute needed, exact-launch arrivals]
 };
 
 __device__ __forceinline__ float as_f(uint32_t x) { return __uint_as_float(x); }
@@ -124,11 +120,7 @@ __device__ __forceinline__ float pair_sum(float x) {
 
 // F8: K/V rows are FP8 E4M3 bytes; staging loads 8 bytes per 8-element
 // piece and widens them exactly to T before the LDS store.
-// EXACT: the bf16 fallback launch. It runs after the main launch on the same
-// stream; its workgroups do nothing unless the main launch raised guard[0].
-// Then every workgroup counts its arrival in guard[1] after reading guard[0];
-// the last one clears both words, so the guard is zero between calls.
-template <typename T, int W, bool QUAD, bool F8, bool EXACT>
+template <typename T, int W, bool QUAD, bool F8>
 __global__ void __launch_bounds__(64 * W, 8 / W)  // two waves per SIMD
 paged_prefill_d128(PrefillArgs<T> a) {
     using SU = std::conditional_t<F8, uint2, U16x8>;  // one staged piece
@@ -147,33 +139,10 @@ paged_prefill_d128(PrefillArgs<T> a) {
     const int col = lane & 31;
     const int half = lane >> 5;
 
-    if constexpr (EXACT) {
-        __shared__ int redo;
-        if (tid == 0) {
-            const int raised = __hip_atomic_load(&a.guard[0], __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-            // A clear guard has nothing to reset: return without counting.
-            // A raised one is seen by every workgroup (it is cleared only
-            // after the last of them has read it and arrived).
-            if (raised) {
-                __threadfence();  // the read completes before the arrival is counted
-                if (atomicAdd(&a.guard[1], 1) == int(gridDim.x) - 1) {  // the last arrival
-                    __hip_atomic_store(&a.guard[1], 0, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(&a.guard[0], 0, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-            redo = raised;
-        }
-        __syncthreads();
-        if (!redo) return;  // uniform
-    }
-
-    // One task = one (item, head, query tile). The main launch has a
-    // workgroup per task; the exact launch, needed only for inputs beyond
-    // fp16's range, loops a few workgroups over all tasks.
-    auto task = [&](int bid) {
+    // The workgroup's task: one (item, head, query tile). Returns whether it
+    // has to be done again with EXACT (see below), for this wave.
+    auto task = [&]<bool EXACT>(std::bool_constant<EXACT>) -> bool {
+        int bid = blockIdx.x;
         // XCD-aware order: hardware deals block ids round-robin over 8 XCDs;
         // give each XCD a contiguous range of logical work.
         if (a.grid % 8 == 0) bid = (bid % 8) * (a.grid / 8) + bid / 8;
@@ -186,7 +155,7 @@ paged_prefill_d128(PrefillArgs<T> a) {
         const int64_t q_begin = a.q_offsets[item];
         const int64_t q_len = a.q_offsets[item + 1] - q_begin;
         const int64_t q0 = int64_t(tile) * BQ;
-        if (q_len <= 0 || q0 >= q_len) return;  // uniform per workgroup
+        if (q_len <= 0 || q0 >= q_len) return false;  // uniform per workgroup
         const int64_t ctx = a.context_lens[item];
         const int64_t first_pos = ctx - q_len;  // absolute position of query 0
         const int64_t table = a.block_offsets[item];
@@ -212,8 +181,12 @@ paged_prefill_d128(PrefillArgs<T> a) {
         // 2^-14, to within 2^-25); a larger, infinite or NaN one becomes an
         // fp16 infinity or NaN, and then so does every output it reaches
         // (p * inf, 0 * inf = NaN; with p <= 2^kSlack and |v| < 65536 the
-        // fp32 sums stay finite otherwise). So a wave whose accumulators end
-        // non-finite raises the guard, and the exact launch redoes the call.
+        // fp32 sums stay finite otherwise). So where a wave's accumulators end
+        // non-finite its workgroup redoes the task with EXACT. (A second
+        // launch that did the whole call again behind a flag cost every call
+        // the launch that found the flag clear: 4 x 512 queries over 2048
+        // tokens, 32 / 8 heads, 78.7 -> 77.3 us; seven prompts of 25-201
+        // tokens, 16 / 8 heads, 19.4 -> 17.7 us, the host's own pace.)
         constexpr bool kConvertV = std::is_same_v<T, __bf16> && !F8 && !EXACT;
 
         const int bs = a.block_size;
@@ -562,16 +535,13 @@ paged_prefill_d128(PrefillArgs<T> a) {
             for (int n = 0; n < 4; ++n)
     #pragma unroll
                 for (int v = 0; v < 16; ++v) total += o[n][v];
-            if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(total) < INFINITY))) {
-                if (lane == 0) a.guard[0] = 1;  // the EXACT launch redoes this call
-                return;
-            }
+            if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(total) < INFINITY))) return true;
         }
-        if (!wave_active) return;
+        if (!wave_active) return false;
 
         const float l = pair_sum(l_run);
         const int64_t qi = wq0 + col;
-        if (qi >= q_len) return;
+        if (qi >= q_len) return false;
         const float inv = a.v_scale / l;
         T* orow = a.out + (q_begin + qi) * a.ots + h * a.ohs + 4 * half;
     #pragma unroll
@@ -583,14 +553,12 @@ paged_prefill_d128(PrefillArgs<T> a) {
                 w.y = pack2<T>(o[n][4 * g + 2] * inv, o[n][4 * g + 3] * inv);
                 *reinterpret_cast<uint2*>(orow + 32 * n + 8 * g) = w;
             }
+        return false;
     };
-    if constexpr (EXACT) {
-        for (int t = blockIdx.x; t < a.grid; t += gridDim.x) {
-            __syncthreads();  // the previous task's LDS reads are done
-            task(t);
-        }
-    } else {
-        task(blockIdx.x);
+    const bool again = task(std::false_type{});
+    if constexpr (std::is_same_v<T, __bf16> && !F8) {
+        // Every wave is past its LDS reads at the barrier.
+        if (__syncthreads_or(again)) task(std::true_type{});  // uniform
     }
 }
 
@@ -600,8 +568,7 @@ paged_prefill_d128(PrefillArgs<T> a) {
 using namespace tvllm;
 
 extern "C" int64_t tvllm_paged_prefill_workspace_size(int dtype, int cache_dtype) {
-    // The fallback guard (two ints) of a bf16 cache, whose V is converted to
-    // fp16 for the P.V products.
+    // Part of the interface (two ints of a bf16 cache's calls); not used.
     return dtype == TVLLM_BF16 && cache_dtype == TVLLM_BF16 ? 2 * int64_t(sizeof(int)) : 0;
 }
 
@@ -728,33 +695,21 @@ extern "C" int tvllm_paged_prefill(
         args.grid = int(grid);
         args.scale_log2 = scale * kLog2e * k_scale;
         args.v_scale = v_scale;
-        args.guard = static_cast<int*>(workspace);
         args.block_shift = (block_size & (block_size - 1)) == 0
                                ? __builtin_ctzll(uint64_t(block_size)) : -1;
         const bool quad = args.block_shift >= 2;
-        auto go = [&]<bool F8, bool EXACT>() {
-            // The exact launch: few workgroups (few arrivals on the guard).
-            const int g = EXACT ? int(std::min<int64_t>(grid, kExactWorkgroups)) : int(grid);
+        auto go = [&]<bool F8>() {
+            const int g = int(grid);
             if (waves == 8) {
-                if (quad) paged_prefill_d128<T, 8, true, F8, EXACT><<<g, 512, 0, s>>>(args);
-                else paged_prefill_d128<T, 8, false, F8, EXACT><<<g, 512, 0, s>>>(args);
+                if (quad) paged_prefill_d128<T, 8, true, F8><<<g, 512, 0, s>>>(args);
+                else paged_prefill_d128<T, 8, false, F8><<<g, 512, 0, s>>>(args);
             } else {
-                if (quad) paged_prefill_d128<T, 4, true, F8, EXACT><<<g, 256, 0, s>>>(args);
-                else paged_prefill_d128<T, 4, false, F8, EXACT><<<g, 256, 0, s>>>(args);
+                if (quad) paged_prefill_d128<T, 4, true, F8><<<g, 256, 0, s>>>(args);
+                else paged_prefill_d128<T, 4, false, F8><<<g, 256, 0, s>>>(args);
             }
         };
-        if (f8) {
-            go.template operator()<true, false>();
-            return launch_status("paged_prefill");
-        }
-        go.template operator()<false, false>();
-        int st = launch_status("paged_prefill");
-        if constexpr (std::is_same_v<T, __bf16>) {
-            if (st == TVLLM_OK) {
-                go.template operator()<false, true>();  // no-op unless V left fp16 range
-                st = launch_status("paged_prefill exact fallback");
-            }
-        }
-        return st;
+        if (f8) go.template operator()<true>();
+        else go.template operator()<false>();
+        return launch_status("paged_prefill");
     });
 }

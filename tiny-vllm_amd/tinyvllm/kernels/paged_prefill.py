@@ -70,7 +70,8 @@ def paged_prefill_attention(
 _GUARDS: dict[tuple[torch.device, int], torch.Tensor] = {}
 _OWNED = threading.local()
 
-# Bytes of the largest fallback guard any call needs (two int32 words).
+# Bytes of the workspace that a call passes along (the library's interface asks
+# for it; its kernels leave it as it is).
 GUARD_BYTES = 8
 
 
@@ -93,8 +94,7 @@ def fallback_guard(guard: torch.Tensor):
 
 def _guard(device: torch.device, nbytes: int) -> torch.Tensor | None:
     """The zero-initialised fallback guard: the one ``fallback_guard``
-    installed, else that of ``device``'s current stream (calls on one stream
-    are ordered, so they can share it; the kernels leave it zero)."""
+    installed, else that of ``device``'s current stream."""
     if nbytes == 0:
         return None
     owned = getattr(_OWNED, "guard", None)
