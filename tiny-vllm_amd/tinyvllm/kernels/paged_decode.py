@@ -2,6 +2,8 @@
 host contract tinyvllm/kernels/paged_decode.cu:469-669)."""
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
 from tinyvllm.kernels._extension import (
@@ -11,11 +13,13 @@ from tinyvllm.paged_kv import PagedKVCache
 from tinyvllm.runtime.contracts import SingleQueryMetadata
 
 
+@lru_cache(maxsize=4096)
 def decode_workspace_bytes(
     num_rows: int, num_heads: int, num_kv_heads: int, head_dim: int,
     max_context_len: int, block_size: int,
 ) -> int:
-    """Split-K scratch the decode kernel needs for this geometry."""
+    """Split-K scratch the decode kernel needs for this geometry (a function
+    of these numbers alone, so the library is asked once for each)."""
     return int(load_kernels().tvllm_paged_decode_workspace_size(
         num_rows, num_heads, num_kv_heads, head_dim, max_context_len, block_size,
     ))
@@ -77,9 +81,8 @@ def paged_decode_attention(
         return
     heads, dim = q.shape[1], q.shape[2]
     max_len = metadata.max_context_len or cache.num_slots
-    need = int(lib.tvllm_paged_decode_workspace_size(
-        num_rows, heads, cache.num_kv_heads, dim, max_len, cache.block_size,
-    ))
+    need = decode_workspace_bytes(num_rows, heads, cache.num_kv_heads, dim, max_len,
+                                  cache.block_size)
     if need and (workspace is None or workspace.numel() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=device)
     check(lib.tvllm_paged_decode(
@@ -156,8 +159,8 @@ def paged_decode_qk_norm_rope(
         return
     heads = q.shape[1]
     max_len = m.max_context_len or cache.num_slots
-    need = int(lib.tvllm_paged_decode_workspace_size(
-        num_rows, heads, cache.num_kv_heads, 128, max_len, cache.block_size))
+    need = decode_workspace_bytes(num_rows, heads, cache.num_kv_heads, 128, max_len,
+                                  cache.block_size)
     if need and (workspace is None or workspace.numel() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=device)
     check(lib.tvllm_paged_decode_qk_norm_rope(
@@ -240,8 +243,8 @@ def paged_decode_qk_norm_rope_partials(
     if num_rows == 0:
         return
     max_len = m.max_context_len or cache.num_slots
-    need = int(lib.tvllm_paged_decode_workspace_size(
-        num_rows, num_heads, cache.num_kv_heads, 128, max_len, cache.block_size))
+    need = decode_workspace_bytes(num_rows, num_heads, cache.num_kv_heads, 128, max_len,
+                                  cache.block_size)
     if need and (workspace is None or workspace.numel() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=device)
     check(lib.tvllm_paged_decode_qk_norm_rope_partials(

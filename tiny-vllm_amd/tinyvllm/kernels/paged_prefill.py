@@ -102,7 +102,7 @@ def _guard(device: torch.device, nbytes: int) -> torch.Tensor | None:
         if owned.device != device or owned.numel() < nbytes:
             raise RuntimeError("the installed fallback guard does not fit this call")
         return owned
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, stream_of(device))
     guard = _GUARDS.get(key)
     if guard is None or guard.numel() < nbytes:
         guard = torch.zeros(nbytes, dtype=torch.uint8, device=device)
