@@ -35,7 +35,7 @@ def test_few_rows_linear(device, rows, pad, columns, width, dtype):
     # Rounding to nearest: half an ulp, itself at most eps times the value.
     tiny = 2.0 ** -24  # fp16 results below its normal range round to this grid
     assert bool(((y.double() - exact).abs() <= slack + ulp / 2 * (exact.abs() + slack) + tiny).all())
-    for slices in (1, 3, 8):
+    for slices in (1, 3, 4, 8):
         parts = few_rows_linear(x, w, slices=slices)
         assert parts.shape == (slices, rows, columns) and parts.dtype == torch.float32
         assert bool(((parts.double().sum(0) - exact).abs() <= slack).all())

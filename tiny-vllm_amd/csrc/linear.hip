@@ -26,6 +26,8 @@
 //   1024 -> 6144 with SiLU  10.5 / 10.9 / 14.7 -> 5.7 / 6.3 / 8.9
 //   2048 -> 1024 partials   4.6 / 6.0 / 5.9 -> 3.2 / 3.5 / 5.0
 //   3072 -> 1024 partials   5.5 / 8.0 / 7.9 -> 3.8 / 4.1 / 6.0
+//   8192 -> 5120 partials   47.6 / 47.6 / 44.5 -> 20.1 / 23.4 / not taken
+//   25600 -> 5120 partials  79.3 / 81.5 / 76.0 -> 60.8 / 71.3 / not taken
 //   4096 -> 24576 with SiLU  47.2 / 46.1 / 50.9 -> 37.2 / 44.4 / 69
 // The last line shows the limit: every workgroup reads the whole input, which
 // past about 16 rows costs large weights more than it saves. The rules of
@@ -227,6 +229,10 @@ extern "C" int tvllm_few_rows_linear(const void* x, int64_t x_row_stride, const 
             if (m <= 16) return go.template operator()<1, 2, 4, 8, kSilu>();
             if (m <= 32) return go.template operator()<2, 2, 4, 4, kSilu>();
             return go.template operator()<4, 2, 2, 4, kSilu>();
+        }
+        if (slices > 0 && n > 2048) {  // enough columns for four waves a workgroup
+            if (m <= 16) return go.template operator()<1, 2, 2, 4, kPartials>();
+            if (m <= 32) return go.template operator()<2, 2, 2, 4, kPartials>();
         }
         if (slices > 0) {
             if (m <= 16) return go.template operator()<1, 2, 2, 8, kPartials>();

@@ -191,20 +191,34 @@ class SplitKLinear(nn.Linear):
             s = 8 if narrow else 4
         return s if self.in_features % (8 * s) == 0 else 1
 
+    def takes_few_rows(self, x: torch.Tensor) -> bool:
+        """Whether a decode batch takes the same slices on the few-rows kernel.
+        Measured on MI355X (bf16, cold weights, us, bmm -> kernel):
+        Up to 2048 columns, eight slices: up to 64 rows with weights of at
+        most 2^22 elements, up to 32 with 13 M. 2048 -> 1024 16 / 64 rows 6.0 /
+        5.9 -> 3.5 / 5.0; 3072 -> 1024 8.0 / 7.9 -> 4.1 / 6.0; 2048 -> 2048 7.0
+        / 7.2 -> 4.5 / 6.5; 6144 -> 2048 16 rows 8.9 -> 8.7, 64 rows 11.6 ->
+        12.8.
+        More columns, four slices: the library's batched product is slow
+        where they are no multiple of 2048 (8192 -> 5120 1-32 rows 48-50 ->
+        20-28; 25600 -> 5120 1 / 24 / 32 rows 79 / 85 / 83.5 -> 61 / 78 /
+        84.5; 4096 -> 2560 1-32 rows 21-24 -> 8-11; past 32 rows it finds
+        better tiles) and as good where they are (4096 -> 4096 1 / 16 rows
+        9.5 / 9.5 -> 8.7 / 9.7; 12288 -> 4096 21.5 / 21.5 -> 22 / 25)."""
+        if x.dim() != 2 or not x.is_contiguous() or self.splits_for(x.shape[0]) == 1:
+            return False  # strided rows take F.linear, as with torch.bmm
+        rows, size = x.shape[0], self.weight.numel()
+        if self.out_features <= 2048:
+            small = size <= (1 << 22 if rows > 32 else 13 << 20)
+        else:
+            small = self.out_features % 2048 != 0 and (
+                rows <= 24 and size <= 1 << 27 or rows <= 32 and size <= 1 << 26)
+        return small and few_rows.fits(x, self.weight)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor | SplitKPartials:
-        # Narrow outputs of a decode batch: the same slices on the few-rows
-        # kernel, up to 64 rows with weights of at most 2^22 elements, up to
-        # 32 with 13 M. Measured on MI355X (eight slices, us, bmm -> kernel):
-        # 2048 -> 1024 16 / 64 rows 6.0 / 5.9 -> 3.5 / 5.0; 3072 -> 1024 8.0 /
-        # 7.9 -> 4.1 / 6.0; 2048 -> 2048 7.0 / 7.2 -> 4.5 / 6.5; 6144 -> 2048
-        # 16 rows 8.9 -> 8.7, 64 rows 11.6 -> 12.8.
-        if (self.out_features <= 2048 and x.dim() == 2
-                and self.weight.numel() <= (1 << 22 if x.shape[0] > 32 else 13 << 20)
-                and few_rows.fits(x, self.weight)):
-            s = self.splits_for(x.shape[0])
-            if s > 1:
-                return SplitKPartials(
-                    few_rows.few_rows_linear(x, self.weight, slices=s), x.dtype)
+        if self.takes_few_rows(x):
+            return SplitKPartials(few_rows.few_rows_linear(
+                x, self.weight, slices=self.splits_for(x.shape[0])), x.dtype)
         # Split-K views the rows in place: only for contiguous 2-D GPU inputs
         # (torch.bmm with an fp32 out_dtype is a GPU-only overload).
         split_ok = x.dim() == 2 and x.is_cuda and x.is_contiguous()
