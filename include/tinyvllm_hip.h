@@ -128,7 +128,7 @@ int64_t tvllm_paged_decode_workspace_size(int64_t num_rows, int64_t num_heads,
 /* The split-K decomposition tvllm_paged_decode uses for this geometry,
  * packed as (waves per KV head << 16) | (workgroups per row << 8) | (KV heads
  * per workgroup) for the MFMA kernel, (1 << 32) | (workgroups per row, KV
- * head and head chunk) for the general kernel (head_dim != 128 or groups
+ * head and head chunk) for the other shapes (head_dim != 128 or groups
  * above 16), 0 for invalid geometry. It depends on max_context_len, so a
  * caller that bakes launches (graph capture) can tell when a tighter context
  * bound would change it. No reference counterpart (the reference kernel has
@@ -148,11 +148,13 @@ int64_t tvllm_paged_decode_split_plan(int64_t num_rows, int64_t num_heads,
  * read - a CSR or pitched per-slot rows), lengths, blocks: int64 device vectors.
  * workspace: >= tvllm_paged_decode_workspace_size(...) bytes (may be NULL
  * when that size is 0). head_dim 128 with group <= 16 and 16-byte aligned
- * rows runs the MFMA kernel; any other head_dim <= 256, group or alignment
- * runs the general kernel (a workgroup of four waves per row, KV head and
- * group of up to 16 query heads, sharing each K/V load; when such units are
- * few, each row's keys split over several workgroups and a second launch
- * merges their partials; fp32 arithmetic, no MFMA).
+ * rows runs the kernel tuned for it; any other head_dim <= 256, group or
+ * alignment runs a workgroup of four waves per row, KV head and group of up
+ * to 16 query heads, sharing each K/V load; when such units are few, each
+ * row's keys split over several workgroups and a second launch merges their
+ * partials. Head dims 32, 64, 128 and 256 with 16-byte aligned cache rows use
+ * MFMAs there too (fp32 sums, weights as two 16-bit terms), others fp32
+ * arithmetic on the vector units.
  * cache_dtype: dtype (caches hold q's element type; k_scale = v_scale = 1)
  * or TVLLM_FP8_E4M3 (caches hold E4M3 bytes in the paged layout;
  * K = stored * k_scale, V = stored * v_scale).
@@ -180,7 +182,7 @@ int tvllm_paged_decode(const void* q, int64_t q_token_stride,
  * split-K partials go to a static 8 MiB device array per GPU (held until
  * the process ends); a geometry whose tvllm_paged_decode_workspace_size
  * exceeds 8 MiB is rejected with TVLLM_EINVAL (the MFMA kernel's split plan
- * needs at most ~6 MB; the general kernel's can need more at head_dim 256
+ * needs at most ~6 MB; that of the other shapes can need more at head_dim 256
  * with groups of 16). Allocates nothing. Calls that
  * overlap on one GPU (different streams) share that array and race; calls
  * ordered on one stream are safe. The first call on a device looks up the
@@ -391,9 +393,11 @@ int tvllm_resolve_tokens(int64_t* tokens, const int64_t* src, const int64_t* pre
  * skipped. max_query_len bounds every item's query length (grid size).
  * cache_dtype / k_scale / v_scale as for tvllm_paged_decode.
  * head_dim 128 runs the MFMA kernel (16-byte aligned Q and cache rows, cache
- * strides in whole 8-element units); any other head_dim <= 256 runs the
- * general kernel of tvllm_paged_decode (fp32; a workgroup per KV head and
- * up to 16 (query token, query head) rows of one item).
+ * strides in whole 8-element units). Any other head_dim <= 256 runs the
+ * kernels that tvllm_paged_decode has for the other shapes: 32, 64 and 256
+ * with 16-byte aligned cache rows on MFMAs (workgroups of 64 or 128 (query
+ * token, query head) rows of one item and KV head, or of up to 16 where an
+ * item has at most 32), others in fp32 (up to 16 rows).
  * workspace: >= tvllm_paged_prefill_workspace_size(dtype, cache_dtype)
  * bytes, 4-byte aligned; left as it is. (A bf16 cache's V is converted to
  * fp16 for the P.V products; a workgroup in which a V value of 65536 or more

@@ -1,7 +1,8 @@
 // Paged attention for any head dim up to 256 (decode rows and prefill
 // chunks), the path behind tvllm_paged_decode and tvllm_paged_prefill for
-// the shapes their MFMA kernels do not take (head_dim != 128, GQA groups
-// above 16, unaligned rows).
+// the shapes their own kernels do not take (head_dim != 128, GQA groups
+// above 16, unaligned rows): on MFMAs at head dims 32, 64, 128 and 256 with
+// vector-aligned cache rows, on the vector units in fp32 otherwise.
 #pragma once
 
 #include "common.h"
@@ -43,7 +44,7 @@ struct GeneralAttention {
     bool q_vec, out_vec;  // query rows in 16-byte pieces, output rows in 8-byte ones
 };
 
-// Grid-level key splits of a decode launch of the general kernel (1: none):
+// Grid-level key splits of a decode launch of these kernels (1: none):
 // enough workgroups to fill the chip when there are few (row, KV head) units,
 // each split keeping at least two rounds of chunks for each of its waves.
 struct GeneralSplits {

@@ -1119,7 +1119,7 @@ extern "C" int64_t tvllm_paged_decode_split_plan(int64_t num_rows, int64_t num_h
         num_heads % num_kv_heads != 0)
         return 0;
     if (head_dim != 128 || num_heads / num_kv_heads > 16) {
-        // The general kernel: its workgroup-level split count, tagged.
+        // general_attention.hip: its workgroup-level split count, tagged.
         const GeneralSplits g = general_decode_splits(num_rows, num_heads, num_kv_heads,
                                                       head_dim, max_context_len);
         return (int64_t(1) << 32) | g.splits;
@@ -1222,9 +1222,9 @@ int paged_decode_impl(
                     "16-byte aligned rows");
         if (!fast) {
             // Other head dims, GQA groups above 16 or unaligned rows: the
-            // general kernel (a workgroup per row, KV head and group of up to
-            // 16 query heads, and split of the keys when there are few of
-            // those; fp32 arithmetic).
+            // kernels of general_attention.hip (a workgroup per row, KV head
+            // and group of up to 16 query heads, and split of the keys when
+            // there are few of those).
             GeneralAttention g{};
             g.q = q;
             g.qts = q_token_stride;

@@ -612,9 +612,8 @@ extern "C" int tvllm_paged_prefill(
                     block_offsets && context_lens,
                 "paged_prefill: null pointer");
     if (head_dim != 128) {
-        // Other head dims: the general kernel (one wave per query token, KV
-        // head and group of up to 16 query heads; fp32 arithmetic, so no
-        // fallback guard is raised).
+        // Other head dims: the kernels of general_attention.hip (32, 64 and 256
+        // on MFMAs, the rest in fp32 on the vector units).
         GeneralAttention g{};
         g.q = q;
         g.qts = q_token_stride;

@@ -8,12 +8,16 @@
 //   top_p (the first token crossing top_p is kept); choice = argmax p / E,
 //   E ~ Exp(1).
 //
-// MI355X design: one 1024-thread workgroup per row, no sort. The kept set is
-// found by radix selection over an order-preserving 32-bit key of s (four
-// 8-bit digit passes, histograms in LDS), weighting each token by its
-// probability mass in 2^-40 fixed point so the sums are exact and
-// deterministic; ties on s are resolved by token index (three more passes),
-// which is exactly the stable sort's order. The noise is a counter-based
+// MI355X design: no sort of a row. Probability masses are 2^-40 fixed point,
+// so every sum is exact and independent of how it is split, and ties on s
+// are resolved by token index, which is exactly the stable sort's order.
+// With the split workspace the vocabulary is cut into spans over the whole
+// chip: row maxima, 2048 bins of the score, the race over the tokens above
+// the cut's bin, and an exact cut of that one bin. Rows that the split does
+// not take, and calls without its workspace, run one 1024-thread workgroup
+// per row: radix selection over an order-preserving 32-bit key of s (four
+// 8-bit digit passes, histograms in LDS, three more for ties). Both keep the
+// same set and draw the same token. The noise is a counter-based
 // Philox4x32-10 stream (Salmon et al., SC'11) keyed by the request seed and
 // its sample counter, so a step is reproducible and graph-capturable.
 #include "common.h"

@@ -78,7 +78,9 @@ GUARD_BYTES = 8
 @contextmanager
 def fallback_guard(guard: torch.Tensor):
     """Calls inside this context use ``guard`` (zero-initialised uint8 of
-    GUARD_BYTES on the calls' device) as their fallback guard. A captured
+    GUARD_BYTES on the calls' device) as the workspace that the C entry asks
+    for (interface only: a workgroup whose V leaves fp16's range redoes its
+    own queries, and nothing is written there any more). A captured
     graph owns its guard this way for the graph's lifetime, instead of one
     keyed by the capture stream's handle, which torch may hand to another
     stream once the capture stream is gone."""

@@ -102,7 +102,9 @@ class PackedLinear(nn.Module):
         (0.6B) 64 rows 11.5 -> 7.3, 32 rows 11.1 -> 6.5, 16 rows 7.4 -> 6.7,
         1 row 7.4 -> 5.5; 4096 -> 6144 (8B) 64 rows 17.8 -> 15.6, 16-32 rows
         and 1 row no gain; 5120 -> 10240 (32B) 64 rows 35.6 -> 25.3, 1-32
-        rows slower. End to end, gains under ~3 us per layer were taken back
+        rows slower. The figures rank the library's two forms: where
+        ``takes_few_rows`` holds (0.6B, say) the caller takes that kernel
+        first. End to end, gains under ~3 us per layer were taken back
         by the decode kernel's prologue (0.6B at 1 and 16 rows: TPOT 1.40 ->
         1.41 and 1.55 -> 1.60 ms; 8B at 64 rows: no change), so only the
         0.6B width at 32-64 rows (C3: 14.9k -> 15.4k tok/s) and widths of

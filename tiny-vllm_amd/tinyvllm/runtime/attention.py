@@ -10,7 +10,8 @@
   * multi-query rows (fresh prompts and chunks with history): MFMA paged
     prefill attention, reading the just-written chunk from the cache too;
   * other head dims (up to 256; the reference dispatches 32, 64, 128, 256)
-    take the same calls, served by the library's general kernel.
+    and GQA groups above 16 take the same calls, served by the library's
+    general_attention.hip (MFMA kernels for those four head dims).
 ``SDPAAttention`` ("reference") is the reference's own torch algorithm
 (gather in logical order + ``F.scaled_dot_product_attention``) kept for
 cross-checking; it is only used when selected explicitly.

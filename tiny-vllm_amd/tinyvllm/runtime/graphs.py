@@ -2,7 +2,7 @@
 (reference: tinyvllm/runtime/graphs.py:12-139).
 
 One graph per batch-size bucket holds the block-table update and token
-resolution -> embedding -> all layers (fused
+resolution (one launch) -> embedding and RoPE rows (one launch) -> all layers (fused
 QK-norm/RoPE/KV-write, split-K paged decode, GEMMs, norms) -> LM head ->
 sampling kernel, reading only the fixed ``DecodeInputs`` views. A replay is
 a single host call, so the per-step host cost no longer scales with
