@@ -82,9 +82,11 @@ def test_unaligned_query_and_output_rows(device, dim, pad):
     assert_bf16_close(out, expect)
 
 
-@pytest.mark.parametrize("dim,group", [(32, 2), (64, 4), (256, 3), (128, 20)])
+@pytest.mark.parametrize("dim,group,dtype", [
+    (32, 2, torch.bfloat16), (64, 4, torch.bfloat16), (256, 3, torch.bfloat16),
+    (128, 20, torch.bfloat16), (64, 4, torch.float16), (256, 3, torch.float16)])
 @pytest.mark.parametrize("longest", [30, 5000])
-def test_decode_with_an_infinite_value(device, dim, group, longest):
+def test_decode_with_an_infinite_value(device, dim, group, dtype, longest):
     """Rows whose V holds an infinity give that infinity (their weights there
     are positive); the other rows and dims are untouched by it."""
     from tinyvllm.kernels.paged_decode import paged_decode_attention
@@ -92,12 +94,12 @@ def test_decode_with_an_infinite_value(device, dim, group, longest):
 
     g = torch.Generator().manual_seed(dim)
     contexts = [longest, 17, 64]
-    cache, k, v, blocks, offsets = _setup(g, contexts, 2, dim, torch.bfloat16, False, device,
+    cache, k, v, blocks, offsets = _setup(g, contexts, 2, dim, dtype, False, device,
                                           "token_major")
     slot = int(blocks[(contexts[0] - 1) // 16]) * 16 + (contexts[0] - 1) % 16
     for t in (v, cache.value[0]):
         t[slot, 1, 3] = float("inf")
-    q = torch.randn(3, 2 * group, dim, generator=g).to(torch.bfloat16)
+    q = torch.randn(3, 2 * group, dim, generator=g).to(dtype)
     rows, lengths = torch.arange(3), torch.tensor(contexts)
     meta = SingleQueryMetadata(rows.to(device), blocks.to(device), offsets.to(device),
                                lengths.to(device), longest)
@@ -110,3 +112,83 @@ def test_decode_with_an_infinite_value(device, dim, group, longest):
     assert torch.equal(torch.isinf(out), torch.isinf(expect))
     finite = torch.isfinite(expect)
     assert_bf16_close(out[finite], expect[finite])
+
+
+def _sink_case(g, lengths, kv_heads, heads, dim, dtype, fp8, gap, device):
+    """Key 0 of every item scores ``gap`` octaves above the others and has
+    V = 0, as an attention sink; the others' scores differ by up to one
+    octave. Stored values, and the context's attention in 64 bits."""
+    pool, blocks, offsets = _pool(g, lengths)
+    k = torch.rand(pool * 16, kv_heads, dim, generator=g)
+    k[..., 1:] *= 0.0
+    v = 64 + 64 * torch.rand(pool * 16, kv_heads, dim, generator=g)
+    a = 4.0  # q = a in dim 0: scores a * k[..., 0], in octaves with this scale
+    scale = math.log(2) / a
+    for i in range(len(lengths)):
+        slot = int(blocks[offsets[i]]) * 16
+        k[slot, :, 0], v[slot] = float(gap), 0.0
+    if fp8:
+        cache, k, v = _fp8_cache(k, v, 16, device, 0.25, 0.5, "head_major")
+    else:
+        k, v = k.to(dtype), v.to(dtype)
+        cache = _Cache(k.to(device), v.to(device), 16, layout="head_major")
+    return cache, k.double(), v.double(), blocks, offsets, a, scale
+
+
+def _sink_bound(dtype, gap):
+    # The result's own rounding; a weight's rounding, at most 2^-36 of the
+    # largest in fp16 and 2^-17 of itself in bf16; exponentials and fp32 sums.
+    own = torch.finfo(dtype).eps / 2
+    return own + (2.0 ** (gap - 36) if dtype == torch.float16 else 2.0 ** -17) + 2.0 ** -15
+
+
+@pytest.mark.parametrize("gap", [12, 20, 24])
+@pytest.mark.parametrize("dim,group,dtype,fp8", [
+    (64, 4, torch.float16, False), (256, 2, torch.float16, False), (32, 1, torch.float16, True),
+    (256, 2, torch.float16, True), (128, 20, torch.float16, False), (64, 4, torch.bfloat16, False)])
+def test_small_weights_beside_a_sink(device, dim, group, dtype, fp8, gap):
+    """Weights far below the row's largest count in full where that one's V is
+    zero: decode (split and unsplit rows) and prefill tiles."""
+    from tinyvllm.kernels.paged_decode import paged_decode_attention
+    from tinyvllm.kernels.paged_prefill import paged_prefill_attention
+    from tinyvllm.runtime.contracts import MultiQueryMetadata, SingleQueryMetadata
+
+    g = torch.Generator().manual_seed(dim + gap)
+    lengths, kv_heads = [3000, 90, 1], 2
+    heads = kv_heads * group
+    cache, k, v, blocks, offsets, a, scale = _sink_case(g, lengths, kv_heads, heads, dim, dtype,
+                                                        fp8, gap, device)
+
+    def exact(item, end):
+        slots = blocks[offsets[item]:offsets[item + 1]].repeat_interleave(16) * 16 \
+            + torch.arange(16).repeat(int(offsets[item + 1] - offsets[item]))
+        slots = slots[:end]
+        w = torch.softmax(k[slots, :, 0] * a * scale, 0)  # [keys, kv_heads]
+        return torch.einsum("kh,khd->hd", w, v[slots]).repeat_interleave(group, 0)
+
+    q = torch.zeros(3, heads, dim, dtype=dtype)
+    q[..., 0] = a
+    rows = torch.arange(3)
+    meta = SingleQueryMetadata(rows.to(device), blocks.to(device), offsets.to(device),
+                               torch.tensor(lengths).to(device), max(lengths))
+    out = torch.zeros_like(q, device=device)
+    paged_decode_attention(q.to(device), cache, 0, meta, out, scale=scale)
+    bound = _sink_bound(dtype, gap)
+    for i in range(3):
+        e = exact(i, lengths[i])
+        assert bool(((out[i].cpu().double() - e).abs() <= bound * e).all()), (i, lengths[i])
+    if dim == 128:
+        return  # prefill at that head dim has a kernel of its own
+    queries = [70, 90, 1]
+    q = torch.zeros(sum(queries), heads, dim, dtype=dtype)
+    q[..., 0] = a
+    starts = torch.tensor([0] + queries).cumsum(0)
+    meta = MultiQueryMetadata(starts.to(device), blocks.to(device), offsets.to(device),
+                              torch.tensor(lengths).to(device), max(queries))
+    out = torch.zeros_like(q, device=device)
+    paged_prefill_attention(q.to(device), cache, 0, meta, out, scale=scale)
+    for i in range(3):
+        for j in (0, queries[i] // 2, queries[i] - 1):
+            e = exact(i, lengths[i] - queries[i] + j + 1)
+            got = out[int(starts[i]) + j].cpu().double()
+            assert bool(((got - e).abs() <= bound * e).all()), (i, j)

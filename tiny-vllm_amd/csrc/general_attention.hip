@@ -220,6 +220,11 @@ __global__ void __launch_bounds__(64) general_attention_kernel(GeneralAttention 
 // in fp32) and the scale is applied in fp32; P enters P.V as two terms of the
 // storage type (P rounded, and the rounded remainder: 16 bits for bf16, 22
 // for fp16), the denominator sums the unrounded P, accumulation is fp32.
+// fp16 has no exponents below 2^-14 and no values below 2^-24: its weights
+// are carried times 2^kLift, which puts the rounding of any of them below
+// 2^-36 of the row's largest (2^-25 without; a row whose largest weight meets
+// V = 0, as attention sinks have it, then came out wrong: its other keys 2^22
+// below the largest 0.3 % off, 2^26 below it zero).
 
 typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gf16x8 __attribute__((ext_vector_type(8)));
@@ -275,26 +280,34 @@ __device__ __forceinline__ float quad_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
+// Weights are 2^(score - m + kLift): fp16's largest, 2^15, are below its
+// 65504. Partial results that leave the kernel (sums and accumulators) state
+// m - kLift as their reference, so that they merge with unlifted ones.
+template <typename T>
+constexpr float kLift = std::is_same_v<T, _Float16> ? 11.f : 0.f;
+template <typename T>
+constexpr float kSlack = std::is_same_v<T, _Float16> ? 4.f : 8.f;
+
 // The online softmax of one step: x holds the lane's scores (base 2, masked
-// ones -inf) and becomes the weights 2^(x - m). The reference m follows the
-// running maximum only once some row of the wave exceeds it by 8: until then
-// the weights stay below 2^8 and nothing needs rescaling. Returns whether it
-// moved; `alpha` is then the factor of what was summed before. Rows with no
-// key yet keep m = -inf and weights 0.
-template <int N>
+// ones -inf) and becomes the weights 2^(x - m + kLift). The reference m
+// follows the running maximum only once some row of the wave exceeds it by
+// kSlack: until then the weights stay below 2^(kSlack + kLift) and nothing
+// needs rescaling. Returns whether it moved; `alpha` is then the factor of
+// what was summed before. Rows with no key yet keep m = -inf and weights 0.
+template <typename T, int N>
 __device__ __forceinline__ bool softmax_step(float (&x)[N], float& m, float& l, float& alpha) {
     float top = x[0];
 #pragma unroll
     for (int i = 1; i < N; ++i) top = fmaxf(top, x[i]);
     top = quad_max(top);
-    const bool moved = __any(top > m + 8.f);  // m = -inf: any key at all
+    const bool moved = __any(top > m + kSlack<T>);  // m = -inf: any key at all
     if (moved) {
         const float mn = fmaxf(m, top);
         alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
         m = mn;
         l *= alpha;
     }
-    const float base = m == -INFINITY ? 0.f : m;
+    const float base = m == -INFINITY ? 0.f : m - kLift<T>;
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -601,7 +614,7 @@ rows_attention_kernel(GeneralAttention a) {
             // and wait for V there.
             __builtin_amdgcn_sched_barrier(0);
             float alpha;
-            if (softmax_step(x, m, l, alpha)) {
+            if (softmax_step<T>(x, m, l, alpha)) {
 #pragma unroll
                 for (int e = 0; e < VE; ++e) acc[e] *= alpha;
             }
@@ -701,7 +714,7 @@ rows_attention_kernel(GeneralAttention a) {
         for (int i = 0; i < 4 * VE; i += 4)
             *reinterpret_cast<float4*>(po + i) = make_float4(o[i], o[i + 1], o[i + 2], o[i + 3]);
         if (quad == 0) {
-            a.part_ml[2 * part] = mx;
+            a.part_ml[2 * part] = mx - kLift<T>;
             a.part_ml[2 * part + 1] = den;
         }
         return;
@@ -946,7 +959,7 @@ tiles_attention_kernel(GeneralAttention a) {
                 for (int i = 0; i < 4; ++i)
                     x[4 * j + i] = 16 * j + i < left ? sc[t][j][i] * qscale : -INFINITY;
             float alpha;
-            if (softmax_step(x, m[t], l[t], alpha)) {
+            if (softmax_step<T>(x, m[t], l[t], alpha)) {
 #pragma unroll
                 for (int d = 0; d < DT; ++d) acc[t][d] *= alpha;
             }
