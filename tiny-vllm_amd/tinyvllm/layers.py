@@ -13,12 +13,23 @@ from collections.abc import Sequence
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as _modules
 
 from tinyvllm._validation import _check_positive_int
 from tinyvllm.kernels import linear as few_rows
 from tinyvllm.kernels.pointwise import (
     add_rms_norm, add_rms_norm_partials, rms_norm, silu_and_mul,
 )
+
+
+def runs_own_forward(module: nn.Module, cls: type[nn.Module]) -> bool:
+    """Whether calling ``module`` is exactly ``cls.forward``: no replacement,
+    subclass or instance ``forward``, and no forward hook, its own or global.
+    A kernel that answers for a module without calling it asks this first."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks
+                     or _modules._global_forward_hooks
+                     or _modules._global_forward_pre_hooks))
 
 
 class PackedLinear(nn.Module):

@@ -25,6 +25,7 @@ from tinyvllm._validation import _check_positive_int
 from tinyvllm.kernels.pointwise import embed_rope, qk_norm_rope
 from tinyvllm.layers import (
     PackedLinear, RMSNorm, RotaryEmbedding, SiluAndMul, SplitKLinear, SplitKPartials,
+    runs_own_forward,
 )
 from tinyvllm.runtime.contracts import AttentionBackend
 
@@ -194,8 +195,8 @@ class Qwen3MLP(nn.Module):
         """Returns SplitKPartials for decode-sized batches (consumed by the
         next RMSNorm.add)."""
         gated = None
-        if not any(m._forward_hooks or m._forward_pre_hooks
-                   for m in (self.gate_up_proj, self.act_fn)):  # only their own calls serve hooks
+        if runs_own_forward(self.gate_up_proj, PackedLinear) and runs_own_forward(
+                self.act_fn, SiluAndMul):
             gated = self.gate_up_proj.gated(hidden_states)
         if gated is None:
             gated = self.act_fn(self.gate_up_proj(hidden_states))
@@ -242,17 +243,17 @@ class Qwen3Model(nn.Module):
     def _embed(self, input_ids: torch.Tensor, positions: torch.Tensor):
         """Embedding rows and (cos, sin) rows of the step's tokens: one launch
         for half-precision tables on the GPU with rows of whole 16-byte units
-        (outside autograd and without hooks, which only the modules' own
-        calls serve), the modules otherwise."""
-        weight = self.embed_tokens.weight
-        if (weight.is_cuda and input_ids.is_cuda and not torch.is_grad_enabled()
+        (outside autograd, with the modules as this class builds them), the
+        modules otherwise."""
+        own = (runs_own_forward(self.embed_tokens, nn.Embedding)
+               and self.embed_tokens.max_norm is None
+               and runs_own_forward(self.rotary_emb, RotaryEmbedding))
+        weight = self.embed_tokens.weight if own else None
+        if (own and weight.is_cuda and input_ids.is_cuda and not torch.is_grad_enabled()
                 and weight.dtype in (torch.float16, torch.bfloat16)
                 and self.config.hidden_size % 8 == 0 and self.config.head_dim % 16 == 0
                 and weight.is_contiguous() and input_ids.is_contiguous()
-                and positions.is_contiguous()
-                and not (self.embed_tokens._forward_hooks or self.embed_tokens._forward_pre_hooks
-                         or self.rotary_emb._forward_hooks
-                         or self.rotary_emb._forward_pre_hooks)):
+                and positions.is_contiguous()):
             hidden, cos, sin = embed_rope(input_ids, positions, weight,
                                           *self.rotary_emb.tables(weight.dtype))
             return hidden, (cos, sin)
