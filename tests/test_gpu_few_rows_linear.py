@@ -64,3 +64,37 @@ def test_layers_take_the_kernel_only_outside_autograd(device):
         torch.testing.assert_close(packed(x), y.detach(), rtol=2 ** -7, atol=2 ** -9)
         assert not packed.takes_few_rows(x[:, ::2][:, :1024].expand(5, 512))
         assert split(x).partials.shape == (8, 5, 1024)
+
+
+def test_tangents_and_transforms_pass_the_projections(device):
+    """no_grad leaves forward-mode AD on, and vmap has no data pointers: both
+    go through torch's ops, as the embedding's rows do."""
+    import torch.autograd.forward_ad as fwad
+    from tinyvllm.layers import PackedLinear, SplitKLinear
+    from tinyvllm.models.qwen3 import Qwen3Config, Qwen3Model
+
+    torch.manual_seed(0)
+    x, t = (torch.randn(4, 1024, device=device, dtype=torch.bfloat16) for _ in range(2))
+    packed = PackedLinear(1024, (512, 512), device=device, dtype=torch.bfloat16)
+    split = SplitKLinear(1024, 1024, device=device, dtype=torch.bfloat16)
+    with torch.no_grad():
+        with fwad.dual_level():
+            y = packed(fwad.make_dual(x, t))
+            tangent = fwad.unpack_dual(y).tangent
+        torch.testing.assert_close(tangent, torch.nn.functional.linear(t, packed.weight))
+        stacked = torch.stack([x, t])
+        y = torch.func.vmap(packed)(stacked)
+        torch.testing.assert_close(y, torch.nn.functional.linear(stacked, packed.weight))
+        assert isinstance(split(x).partials, torch.Tensor)
+        config = Qwen3Config(
+            vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1,
+            max_position_embeddings=32, num_attention_heads=2, num_key_value_heads=1, head_dim=32,
+            rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=True)
+        model = Qwen3Model(config, device=device, dtype=torch.bfloat16)
+        ids, positions = torch.tensor([3, 5], device=device), torch.tensor([0, 1], device=device)
+        weight = model.embed_tokens.weight
+        del model.embed_tokens.weight
+        with fwad.dual_level():
+            model.embed_tokens.weight = fwad.make_dual(weight.detach(), torch.ones_like(weight))
+            hidden, _ = model._embed(ids, positions)
+            assert bool((fwad.unpack_dual(hidden).tangent == 1).all())

@@ -17,6 +17,9 @@ from functools import lru_cache
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 LIBRARY_PATH = Path(__file__).resolve().parent / "libtinyvllm_hip.so"
 ABI_VERSION = 5
@@ -161,3 +164,20 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
         if tensor.get_device() != index:
             raise RuntimeError("tensors must share one GPU device")
     return device
+
+
+def values_only(*tensors: torch.Tensor) -> bool:
+    """Whether a call asks for these tensors' values and nothing else, which is
+    all that a kernel behind the C interface gives: no gradient, no
+    forward-mode tangent (no_grad leaves those on), no vmap or other function
+    transform, no tracing or compilation, no dispatch or function mode that
+    wants to see torch's ops, no tensor subclass. A module that has a torch
+    form too takes it otherwise."""
+    return not (
+        torch.compiler.is_compiling() or torch.is_grad_enabled()
+        or forward_ad._current_level >= 0
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+        or (torch._C._len_torch_function_stack() > 0
+            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+    ) and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)

@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from tinyvllm.kernels._extension import (
-    check, dtype_code, load_kernels, require_gpu, stream_of,
+    check, dtype_code, load_kernels, require_gpu, stream_of, values_only,
 )
 
 MAX_ROWS = 64
@@ -14,10 +14,11 @@ MAX_ROWS = 64
 def fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``few_rows_linear`` takes these tensors: 1 to 64 half-precision
     rows on the GPU in 16-byte units, widths in multiples of 32, outside
-    autograd and autocast (which only the torch ops serve)."""
-    return (x.dim() == 2 and x.is_cuda and x.dtype == weight.dtype
+    autocast and wherever more than values is asked for (autograd, forward
+    mode, transforms, tracing), which only the torch ops serve."""
+    return (values_only(x, weight) and x.dim() == 2 and x.is_cuda and x.dtype == weight.dtype
             and x.dtype in (torch.bfloat16, torch.float16) and 0 < x.shape[0] <= MAX_ROWS
-            and weight.device == x.device and not torch.is_grad_enabled()
+            and weight.device == x.device
             and not torch.is_autocast_enabled("cuda")
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.is_contiguous()
             and weight.shape[0] % 32 == 0 and weight.shape[1] % 32 == 0

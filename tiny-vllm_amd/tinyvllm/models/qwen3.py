@@ -22,6 +22,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from tinyvllm._validation import _check_positive_int
+from tinyvllm.kernels._extension import values_only
 from tinyvllm.kernels.pointwise import embed_rope, qk_norm_rope
 from tinyvllm.layers import (
     PackedLinear, RMSNorm, RotaryEmbedding, SiluAndMul, SplitKLinear, SplitKPartials,
@@ -243,13 +244,14 @@ class Qwen3Model(nn.Module):
     def _embed(self, input_ids: torch.Tensor, positions: torch.Tensor):
         """Embedding rows and (cos, sin) rows of the step's tokens: one launch
         for half-precision tables on the GPU with rows of whole 16-byte units
-        (outside autograd, with the modules as this class builds them), the
-        modules otherwise."""
+        (where only values are asked for, with the modules as this class builds
+        them), the modules otherwise."""
         own = (runs_own_forward(self.embed_tokens, nn.Embedding)
                and self.embed_tokens.max_norm is None
                and runs_own_forward(self.rotary_emb, RotaryEmbedding))
         weight = self.embed_tokens.weight if own else None
-        if (own and weight.is_cuda and input_ids.is_cuda and not torch.is_grad_enabled()
+        if (own and weight.is_cuda and input_ids.is_cuda
+                and values_only(weight, input_ids, positions)
                 and weight.dtype in (torch.float16, torch.bfloat16)
                 and self.config.hidden_size % 8 == 0 and self.config.head_dim % 16 == 0
                 and weight.is_contiguous() and input_ids.is_contiguous()
