@@ -61,3 +61,22 @@ def test_begin_decode_equals_its_two_ops(device, rows, count):
             resolve_tokens(tokens, src, prev)
         results.append((table.clone(), tokens.clone()))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_unaligned_embedding_takes_the_modules(device):
+    """A table that starts off a 16-byte boundary (a view into a larger
+    buffer) gives its rows all the same."""
+    from tinyvllm.models.qwen3 import Qwen3Config, Qwen3Model
+
+    config = Qwen3Config(
+        vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1,
+        max_position_embeddings=32, num_attention_heads=2, num_key_value_heads=1, head_dim=32,
+        rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=True)
+    model = Qwen3Model(config, device=device, dtype=torch.bfloat16)
+    flat = torch.randn(1 + 64 * 64, device=device).to(torch.bfloat16)
+    model.embed_tokens.weight = torch.nn.Parameter(flat[1:].view(64, 64))
+    ids, positions = torch.tensor([3, 63], device=device), torch.tensor([0, 31], device=device)
+    with torch.no_grad():
+        hidden, (cos, _) = model._embed(ids, positions)
+    assert torch.equal(hidden, flat[1:].view(64, 64)[ids])
+    assert torch.equal(cos, model.rotary_emb.tables(torch.bfloat16)[0][positions][:, None])

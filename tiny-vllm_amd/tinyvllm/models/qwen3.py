@@ -243,22 +243,23 @@ class Qwen3Model(nn.Module):
 
     def _embed(self, input_ids: torch.Tensor, positions: torch.Tensor):
         """Embedding rows and (cos, sin) rows of the step's tokens: one launch
-        for half-precision tables on the GPU with rows of whole 16-byte units
-        (where only values are asked for, with the modules as this class builds
-        them), the modules otherwise."""
-        own = (runs_own_forward(self.embed_tokens, nn.Embedding)
-               and self.embed_tokens.max_norm is None
-               and runs_own_forward(self.rotary_emb, RotaryEmbedding))
-        weight = self.embed_tokens.weight if own else None
-        if (own and weight.is_cuda and input_ids.is_cuda
-                and values_only(weight, input_ids, positions)
-                and weight.dtype in (torch.float16, torch.bfloat16)
-                and self.config.hidden_size % 8 == 0 and self.config.head_dim % 16 == 0
-                and weight.is_contiguous() and input_ids.is_contiguous()
-                and positions.is_contiguous()):
-            hidden, cos, sin = embed_rope(input_ids, positions, weight,
-                                          *self.rotary_emb.tables(weight.dtype))
-            return hidden, (cos, sin)
+        for half-precision tables on the GPU, aligned and with rows of whole
+        16-byte units (where only values are asked for, with the modules as
+        this class builds them), the modules otherwise."""
+        if (runs_own_forward(self.embed_tokens, nn.Embedding)
+                and self.embed_tokens.max_norm is None
+                and runs_own_forward(self.rotary_emb, RotaryEmbedding)):
+            weight = self.embed_tokens.weight
+            if (weight.is_cuda and input_ids.is_cuda
+                    and values_only(weight, input_ids, positions)
+                    and weight.dtype in (torch.float16, torch.bfloat16)
+                    and self.config.hidden_size % 8 == 0 and self.config.head_dim % 16 == 0
+                    and weight.is_contiguous() and input_ids.is_contiguous()
+                    and positions.is_contiguous()):
+                tables = self.rotary_emb.tables(weight.dtype)
+                if all(t.data_ptr() % 16 == 0 for t in (weight, *tables)):
+                    hidden, cos, sin = embed_rope(input_ids, positions, weight, *tables)
+                    return hidden, (cos, sin)
         hidden = self.embed_tokens(input_ids)
         return hidden, self.rotary_emb(positions, hidden.dtype)
 
