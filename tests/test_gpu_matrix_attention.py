@@ -82,6 +82,43 @@ def test_unaligned_query_and_output_rows(device, dim, pad):
     assert_bf16_close(out, expect)
 
 
+@pytest.mark.parametrize("dim", [32, 64, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fp8_rows_at_8_byte_boundaries(device, dim, dtype):
+    """FP8 cache rows 8 bytes off every 16-byte boundary, decode and prefill."""
+    from tinyvllm.kernels.paged_decode import paged_decode_attention
+    from tinyvllm.runtime.contracts import SingleQueryMetadata
+
+    g = torch.Generator().manual_seed(dim)
+    contexts, kv_heads = [300, 17, 64], 2
+    aligned, k, v, blocks, offsets = _setup(g, contexts, kv_heads, dim, dtype, True, device,
+                                            "token_major")
+    slots, row = aligned.num_slots, kv_heads * dim + 24
+
+    def shifted(t):
+        bytes_ = torch.zeros(slots * row + 8, dtype=torch.uint8, device=device)
+        view = bytes_[8:].view(slots, row)[:, :kv_heads * dim].unflatten(1, (kv_heads, dim))
+        view.copy_(t.view(torch.uint8))
+        return view.view(torch.float8_e4m3fn)
+
+    cache = _Cache(shifted(aligned.key[0]), shifted(aligned.value[0]), 16, 0.5, 2.0,
+                   layout="token_major")
+    assert cache.key[0].data_ptr() % 16 == 8 and cache.key[0].stride(0) % 16 == 8
+    q = torch.randn(3, 4 * kv_heads, dim, generator=g).to(dtype)
+    rows, lengths = torch.arange(3), torch.tensor(contexts)
+    meta = SingleQueryMetadata(rows.to(device), blocks.to(device), offsets.to(device),
+                               lengths.to(device), max(contexts))
+    out = torch.zeros(q.shape, dtype=dtype, device=device)
+    paged_decode_attention(q.to(device), cache, 0, meta, out, scale=dim ** -0.5)
+    expect = torch.zeros(q.shape, dtype=dtype)
+    OA.decode_attention(q, k, v, rows, blocks, offsets, lengths, 16, dim ** -0.5, expect)
+    assert_bf16_close(out, expect)
+    queries = [30, 17, 1]
+    q = torch.randn(sum(queries), 4 * kv_heads, dim, generator=g).to(dtype)
+    out, expect = _prefill(device, q, cache, k, v, blocks, offsets, queries, contexts, dim)
+    assert_bf16_close(out, expect)
+
+
 @pytest.mark.parametrize("dim,group,dtype", [
     (32, 2, torch.bfloat16), (64, 4, torch.bfloat16), (256, 3, torch.bfloat16),
     (128, 20, torch.bfloat16), (64, 4, torch.float16), (256, 3, torch.float16)])

@@ -270,6 +270,11 @@ __device__ __forceinline__ void split_p(const float (&p)[8], U16x8& hi, U16x8& l
     }
 }
 
+// 16 bytes at an 8-byte boundary.
+struct alignas(8) U16x8Half {
+    uint32_t w[4];
+};
+
 // Max / sum over the four quads that share a query row.
 __device__ __forceinline__ float quad_max(float v) {
     v = fmaxf(v, __shfl_xor(v, 16, 64));
@@ -558,9 +563,11 @@ rows_attention_kernel(GeneralAttention a) {
                     vreg[j][i][0] = x.x;
                     vreg[j][i][1] = x.y;
                 } else {
+                    // FP8 rows are 8-byte aligned only.
+                    using V16 = std::conditional_t<F8, U16x8Half, U16x8>;
 #pragma unroll
                     for (int w = 0; w < VB / 16; ++w) {
-                        const U16x8 x = *reinterpret_cast<const U16x8*>(p + 16 * w);
+                        const V16 x = *reinterpret_cast<const V16*>(p + 16 * w);
 #pragma unroll
                         for (int y = 0; y < 4; ++y) vreg[j][i][4 * w + y] = x.w[y];
                     }
