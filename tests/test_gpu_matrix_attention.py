@@ -82,6 +82,26 @@ def test_unaligned_query_and_output_rows(device, dim, pad):
     assert_bf16_close(out, expect)
 
 
+def test_longest_chunks_of_wide_groups(device):
+    """65535 queries of 128 heads on one KV head: more row tiles than a grid
+    dimension holds (the bound alone; the items themselves are short)."""
+    from tinyvllm.kernels.paged_prefill import paged_prefill_attention
+    from tinyvllm.runtime.contracts import MultiQueryMetadata
+
+    g = torch.Generator().manual_seed(1)
+    cache, k, v, blocks, offsets = _setup(g, [40, 3], 1, 256, torch.bfloat16, False, device,
+                                          "token_major")
+    q = torch.randn(7, 128, 256, generator=g).to(torch.bfloat16)
+    starts, lengths = torch.tensor([0, 5, 7]), torch.tensor([40, 3])
+    meta = MultiQueryMetadata(starts.to(device), blocks.to(device), offsets.to(device),
+                              lengths.to(device), 65535)
+    out = torch.zeros_like(q, device=device)
+    paged_prefill_attention(q.to(device), cache, 0, meta, out, scale=256 ** -0.5)
+    expect = torch.zeros_like(q)
+    OA.prefill_attention(q, k, v, starts, blocks, offsets, lengths, 16, 256 ** -0.5, expect)
+    assert_bf16_close(out, expect)
+
+
 @pytest.mark.parametrize("dim", [32, 64, 256])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fp8_rows_at_8_byte_boundaries(device, dim, dtype):

@@ -1167,7 +1167,14 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     // Prefill (head dim 128 has its own kernel): the tiled kernel from 32 rows per item and KV head (where two
     // of its waves have rows); below, four waves share the keys of 16 rows.
     const int64_t item_rows = g.max_query_len * group;
-    const bool tiles = rows_kernel && D != 128 && !g.rows && item_rows > 2 * GH;
+    const int64_t units = g.num_items * g.kv_heads;
+    // 128 rows per workgroup where that leaves one for every CU (4 x 512
+    // queries over 2048 tokens, 32 / 8 heads of 64: 84 us against 99 with 64
+    // rows; heads of 256 gain nothing, 320 against 329, and lose where tiles
+    // are few, 72 against 63 us for 3 x 300).
+    const bool wide = D <= 64 && units * ((item_rows + 127) / 128) >= 256;
+    const int64_t ty = (item_rows + (wide ? 127 : 63)) / (wide ? 128 : 64);
+    const bool tiles = rows_kernel && D != 128 && !g.rows && item_rows > 2 * GH && ty <= 65535;
     g.splits = 1;
     g.split_keys = 0;
     g.part_o = g.part_ml = nullptr;
@@ -1193,19 +1200,11 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     return dispatch_half(g.dtype, [&]<int DT>() {
         using T = typename Elem<DT>::T;
         if (tiles) {
-            // 128 rows per workgroup where that leaves one for every CU (4 x
-            // 512 queries over 2048 tokens, 32 / 8 heads of 64: 84 us against
-            // 99 with 64 rows; heads of 256 gain nothing, 320 against 329, and
-            // lose where tiles are few, 72 against 63 us for 3 x 300). Where
-            // 64 rows do not fill the CUs either, two halves of a workgroup
+            // Where the tiles do not fill the CUs, two halves of a workgroup
             // share the keys (2 x 256 over 1033, heads of 256: 61 -> 53 us; 8
             // x 40 over 2040, FP8, heads of 64: 43 -> 35 us); at full grids
             // the halves only add their merge (99 -> 112 us).
-            const int64_t units = g.num_items * g.kv_heads;
-            const bool wide = D <= 64 && units * ((item_rows + 127) / 128) >= 256;
-            const int64_t ty = (item_rows + (wide ? 127 : 63)) / (wide ? 128 : 64);
             const bool halves = units * ty < 256;
-            TVLLM_CHECK(units <= INT32_MAX && ty <= 65535, "attention: launch grid out of range");
             const dim3 tg{static_cast<uint32_t>(units), static_cast<uint32_t>(ty), 1u};
             auto go = [&]<int DD, int RT, int HV>() {
                 constexpr int threads = 64 * kRowWaves * HV;
