@@ -32,6 +32,86 @@ def runs_own_forward(module: nn.Module, cls: type[nn.Module]) -> bool:
                      or _modules._global_forward_pre_hooks))
 
 
+# Most rows at which the few-rows kernel takes a projection [columns, width]
+# from the library, by its three forms. Measured on MI355X in graph replay over
+# cold weights (bf16, 1-64 rows, widths 64-25600, columns 64-32768: some 4000
+# points; inside the limits the kernel was never more than 3 % or 0.1 us the
+# slower). Every workgroup reads all the rows, so the limit falls with the
+# width; few columns leave CUs idle; the exceptions at wide columns are the
+# library's good and bad tiles.
+
+def _rounded_limit(columns: int, width: int) -> int:
+    """Against F.linear. us, library -> kernel: 1024 -> 4096 1 / 16 / 64 rows 7.3 /
+    7.4 / 11.4 -> 4.0 / 4.5 / 7.1; 2048 -> 4096 16 / 32 rows 11.4 / 11.6 -> 6.5 /
+    8.0; 4096 -> 2048 16 / 24 / 32 rows 14.5 / 14.5 / 11.9 -> 10.1 / 11.9 / 13.2;
+    5120 -> 1536 8 / 16 rows 17.9 / 10.1 -> 11.7 / 13.5; 6144 -> 1024 1 row 10.3 ->
+    11.1; 256 -> 32768 32 rows 7.3 -> 9.9."""
+    if columns * width > 1 << 23 or columns > 32768 or columns < 256 and width > 1024:
+        return 0
+    if width <= 1024:
+        if columns <= 8192 and columns * width <= 1 << 22:
+            return 64
+        return 32 if columns <= 16384 else 16
+    if width <= 2048:
+        if columns > 4096:
+            return 16
+        return 64 if columns >= 1536 and columns * width <= 1 << 22 else 32
+    if width <= 4096:
+        return 24 if columns >= 512 else 16
+    return 8 if width <= 5120 else 0
+
+
+def _gated_limit(columns: int, width: int) -> int:
+    """Against F.linear and silu_and_mul (columns: gate and up). us: 1024 -> 6144
+    16 / 64 rows 10.7 / 14.5 -> 6.0 / 8.5; 2048 -> 12288 16 / 32 rows 17.6 / 17.7
+    -> 16.5 / 19.6; 2560 -> 19456 16 rows 49.6 -> 33.6, but 2560 -> 16384 21.8 ->
+    25.8; 4096 -> 24576 1 / 16 rows 45.9 / 46.6 -> 37.9 / 45.1; 8192 -> 1024 1 row
+    14.0 -> 21.8; 5120 -> 51200 1 row 91.7 -> 127."""
+    if columns > 32768 or width > 4096:
+        return 0
+    small = columns * width <= 1 << 23
+    if width <= 1024:
+        return 64 if small else 16
+    if width <= 2048:
+        if small:
+            return 64 if columns >= 1536 else 32 if columns >= 768 else 16
+        wide = 8192 < columns <= 16384 or columns > 24576
+        return 8 if wide and width < 2048 else 16
+    if columns < 512:
+        return 0
+    if columns <= 8192 or width == 4096:
+        return 16
+    return 16 if 16384 < columns <= 24576 and width <= 3072 else 0
+
+
+def _partials_limit(columns: int, width: int) -> int:
+    """Against the batched product over as many slices (eight up to 2048 columns,
+    four above). us: 2048 -> 1024 16 / 64 rows 6.3 / 6.3 -> 3.4 / 4.8; 3072 -> 1024
+    7.8 / 7.8 -> 3.9 / 5.8; 1024 -> 2048 64 rows 5.4 -> 7.2; 6144 -> 2048 16 rows 8.7
+    -> 9.1; 53248 -> 256 32 rows 12.0 -> 29.9. More columns: the library is slow
+    where they are no multiple of 2048 (8192 -> 5120 1 / 32 rows 48 / 49 -> 20 / 28;
+    25600 -> 5120 1 / 24 / 32 rows 81 / 85 / 85 -> 62 / 79 / 85; 4096 -> 2560 1 / 32
+    rows 24 / 21 -> 8 / 10; past 32 rows it finds better tiles; 9728 -> 7168 24 rows 33.6
+    -> 47.0) and as good where they are (4096 -> 4096 1 / 16 rows 9.5 / 9.5 -> 8.7 /
+    9.7; 12288 -> 4096 21.5 / 21.5 -> 22 / 25)."""
+    size = columns * width
+    if columns <= 2048:
+        if size > (13 << 20 if columns <= 1536 else 1 << 23) or columns < 256 and width > 6144:
+            return 0
+        if width > 12288 or width < 512 and columns > 1024:
+            return 16
+        if 1024 <= width <= 4096 and columns <= 1024:
+            return 64
+        return 24 if width > 4096 and columns <= 512 else 32
+    if columns % 2048 == 0 or columns > 7168 or width > 25600 or size > 1 << 27:
+        return 0
+    if columns > 5120:
+        return 32 if width <= 4096 else 0
+    if width > 12288:
+        return 16 if columns <= 3072 else 24 if columns >= 4096 else 0
+    return 32
+
+
 class PackedLinear(nn.Module):
     """Bias-free linear layer whose output rows pack several named shards
     (q|k|v, gate|up), so one GEMM serves them all (reference layers.py:19-125)."""
@@ -76,28 +156,16 @@ class PackedLinear(nn.Module):
         return F.linear(x, self.weight)
 
     def takes_few_rows(self, x: torch.Tensor) -> bool:
-        """Whether this call runs on the few-rows kernel: up to 64 rows with a
-        weight of at most 2^22 elements, up to 32 with 2^23. Measured on
-        MI355X (bf16, cold weights, us, F.linear -> kernel): 1024 -> 4096
-        (2^22) 16 rows 7.6 -> 4.6, 64 rows 11.6 -> 7.4; 2048 -> 4096 (2^23)
-        16 rows 11.7 -> 6.7, 32 rows 11.9 -> 8.3, 64 rows 12.4 -> 12.1; 4096
-        -> 6144 16 rows 14.4 -> 15.7, 64 rows 17.8 -> 25.7."""
-        limit = 1 << (22 if x.dim() == 2 and x.shape[0] > 32 else 23)
-        return self.weight.numel() <= limit and few_rows.fits(x, self.weight)
+        """Whether this call runs on the few-rows kernel."""
+        return (x.dim() == 2 and x.shape[0] <= _rounded_limit(*self.weight.shape)
+                and few_rows.fits(x, self.weight))
 
     def gated(self, x: torch.Tensor) -> torch.Tensor | None:
         """silu(gate) * up of a [gate | up] projection in one launch, or None
-        where the projection and the activation on their own are faster: up
-        to 16 rows with weights of at most 2^27 elements, up to 64 with 2^23.
-        Measured on MI355X (bf16, cold weights, us, F.linear + silu_and_mul
-        -> kernel): 1024 -> 6144 16 / 64 rows 10.9 / 14.7 -> 6.3 / 8.9; 2048
-        -> 12288 16 rows 18.1 -> 16.1, 32 rows 18.1 -> 19.5; 4096 -> 24576 1
-        / 16 rows 47.2 / 46.1 -> 37.2 / 44.4, 64 rows 50.9 -> 73; 5120 ->
-        51200 1 row 91.7 -> 127."""
-        if len(self.output_sizes) != 2 or self.output_sizes[0] != self.output_sizes[1]:
-            return None
-        limit = 1 << (23 if x.dim() == 2 and x.shape[0] > 16 else 27)
-        if (self.weight.numel() > limit or self.output_sizes[0] % 16
+        where the projection and the activation on their own are faster."""
+        if (len(self.output_sizes) != 2 or self.output_sizes[0] != self.output_sizes[1]
+                or self.output_sizes[0] % 16 or x.dim() != 2
+                or x.shape[0] > _gated_limit(*self.weight.shape)
                 or not few_rows.fits(x, self.weight)):
             return None
         return few_rows.few_rows_linear(x, self.weight, silu=True)
@@ -205,28 +273,11 @@ class SplitKLinear(nn.Linear):
         return s if self.in_features % (8 * s) == 0 else 1
 
     def takes_few_rows(self, x: torch.Tensor) -> bool:
-        """Whether a decode batch takes the same slices on the few-rows kernel.
-        Measured on MI355X (bf16, cold weights, us, bmm -> kernel):
-        Up to 2048 columns, eight slices: up to 64 rows with weights of at
-        most 2^22 elements, up to 32 with 13 M. 2048 -> 1024 16 / 64 rows 6.0 /
-        5.9 -> 3.5 / 5.0; 3072 -> 1024 8.0 / 7.9 -> 4.1 / 6.0; 2048 -> 2048 7.0
-        / 7.2 -> 4.5 / 6.5; 6144 -> 2048 16 rows 8.9 -> 8.7, 64 rows 11.6 ->
-        12.8.
-        More columns, four slices: the library's batched product is slow
-        where they are no multiple of 2048 (8192 -> 5120 1-32 rows 48-50 ->
-        20-28; 25600 -> 5120 1 / 24 / 32 rows 79 / 85 / 83.5 -> 61 / 78 /
-        84.5; 4096 -> 2560 1-32 rows 21-24 -> 8-11; past 32 rows it finds
-        better tiles) and as good where they are (4096 -> 4096 1 / 16 rows
-        9.5 / 9.5 -> 8.7 / 9.7; 12288 -> 4096 21.5 / 21.5 -> 22 / 25)."""
-        if x.dim() != 2 or not x.is_contiguous() or self.splits_for(x.shape[0]) == 1:
-            return False  # strided rows take F.linear, as with torch.bmm
-        rows, size = x.shape[0], self.weight.numel()
-        if self.out_features <= 2048:
-            small = size <= (1 << 22 if rows > 32 else 13 << 20)
-        else:
-            small = self.out_features % 2048 != 0 and (
-                rows <= 24 and size <= 1 << 27 or rows <= 32 and size <= 1 << 26)
-        return small and few_rows.fits(x, self.weight)
+        """Whether a decode batch takes the same slices on the few-rows kernel
+        (strided rows take F.linear, as with torch.bmm)."""
+        return (x.dim() == 2 and x.is_contiguous() and self.splits_for(x.shape[0]) > 1
+                and x.shape[0] <= _partials_limit(*self.weight.shape)
+                and few_rows.fits(x, self.weight))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor | SplitKPartials:
         if self.takes_few_rows(x):
