@@ -249,3 +249,126 @@ def test_small_weights_beside_a_sink(device, dim, group, dtype, fp8, gap):
             e = exact(i, lengths[i] - queries[i] + j + 1)
             got = out[int(starts[i]) + j].cpu().double()
             assert bool(((got - e).abs() <= bound * e).all()), (i, j)
+
+
+def _with_specials(cache, specials, contexts, blocks, offsets, device, run):
+    """Two runs over the same cache: V zero at the special elements (item, key,
+    kv head, dim, value), then holding them; the plain run's output with what
+    the specials make of it, and the special run's."""
+    value = cache.value[0]
+
+    def place(zero):
+        for item, key, head, d, x in specials:
+            slot = int(blocks[offsets[item] + key // 16]) * 16 + key % 16
+            value[slot, head, d] = torch.tensor(0.0 if zero else x).to(value.dtype).to(device)
+
+    place(True)
+    plain = run()
+    place(False)
+    return plain, run()
+
+
+def _expect(plain, specials, rows_seeing, group):
+    """rows_seeing(item, key): the output rows whose queries see the key."""
+    expect = plain.clone().float()
+    for item, key, head, d, x in specials:
+        for r in rows_seeing(item, key):
+            expect[r, head * group:(head + 1) * group, d] += x
+    return expect.to(plain.dtype)
+
+
+def _assert_same(out, expect):
+    assert torch.equal(out.isnan(), expect.isnan())
+    finite_or_inf = ~expect.isnan()
+    assert torch.equal(out[finite_or_inf], expect[finite_or_inf])
+
+
+INF, NAN = float("inf"), float("nan")
+
+
+@pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False),
+                                       (torch.float16, True)])
+@pytest.mark.parametrize("dim,kv_heads,group,items", [
+    (64, 2, 2, [(8, 31), (5, 60)]),          # up to 16 rows: rows kernel, several queries each
+    (256, 2, 1, [(30, 400), (3, 3)]),        # rows kernel
+    (32, 1, 1, [(64, 64), (129, 400)]),      # 64-row tiles, two halves
+    (64, 2, 3, [(65, 97), (70, 300)]),       # two halves
+    (256, 2, 2, [(40, 40), (100, 333)]),     # two halves
+    (64, 8, 1, [(100, 150)] * 18),           # 64-row tiles, one half
+    (256, 8, 4, [(60, 130)] * 9),            # one half
+    (32, 8, 8, [(77, 200)] * 7 + [(2, 65)]), # 128-row tiles
+    (64, 8, 8, [(77, 200)] * 7 + [(40, 40)])])
+def test_prefill_with_infinities_and_nans(device, dim, kv_heads, group, items, dtype, fp8):
+    """Queries before a key whose V holds an infinity or a NaN keep their bits;
+    later ones get it in its dim alone."""
+    g = torch.Generator().manual_seed(dim + group)
+    queries, contexts = [list(x) for x in zip(*items)]
+    cache, k, v, blocks, offsets = _setup(g, contexts, kv_heads, dim, dtype, fp8, device,
+                                          "token_major")
+    q = torch.randn(sum(queries), kv_heads * group, dim, generator=g).to(dtype)
+    starts = [0]
+    for n in queries:
+        starts.append(starts[-1] + n)
+
+    def middle(item):  # a key that about half of the item's queries see
+        return contexts[item] - 1 - queries[item] // 2
+
+    specials = [(0, middle(0), 0, 3, NAN), (1, middle(1), kv_heads - 1, dim - 1, NAN)]
+    if not fp8:
+        specials = [(0, middle(0), 0, 3, INF), (0, middle(0), 0, 17, -INF),
+                    (0, contexts[0] - 1, 0, 17, INF), (1, middle(1), kv_heads - 1, dim - 1, NAN),
+                    (1, 0, 0, 0, -INF)]
+
+    def run():
+        return _prefill(device, q, cache, k, v, blocks, offsets, queries, contexts, dim)[0]
+
+    def seeing(item, key):
+        first = max(0, key - (contexts[item] - queries[item]))
+        return range(starts[item] + first, starts[item + 1])
+
+    plain, out = _with_specials(cache, specials, contexts, blocks, offsets, device, run)
+    _assert_same(out, _expect(plain, specials, seeing, group))
+
+
+@pytest.mark.parametrize("dim,group,dtype,fp8", [
+    (32, 2, torch.bfloat16, True), (64, 4, torch.bfloat16, False), (64, 4, torch.float16, False),
+    (256, 3, torch.float16, True), (256, 16, torch.bfloat16, False),
+    (128, 20, torch.bfloat16, False)])
+@pytest.mark.parametrize("contexts", [[30, 17], [5000, 300, 1], [700] * 40])
+def test_decode_with_infinities_and_nans(device, dim, group, dtype, fp8, contexts):
+    from tinyvllm.kernels.paged_decode import paged_decode_attention
+    from tinyvllm.runtime.contracts import SingleQueryMetadata
+
+    g = torch.Generator().manual_seed(dim)
+    cache, _, _, blocks, offsets = _setup(g, contexts, 2, dim, dtype, fp8, device, "head_major")
+    n = len(contexts)
+    q = torch.randn(n, 2 * group, dim, generator=g).to(dtype).to(device)
+    meta = SingleQueryMetadata(torch.arange(n).to(device), blocks.to(device), offsets.to(device),
+                               torch.tensor(contexts).to(device), max(contexts))
+    x = NAN if fp8 else -INF
+    specials = [(0, contexts[0] - 1, 0, 3, x), (1, 0, 1, dim - 1, NAN),
+                (1, contexts[1] // 2, 0, dim // 2, x)]
+
+    def run():
+        out = torch.zeros_like(q)
+        paged_decode_attention(q, cache, 0, meta, out, scale=dim ** -0.5)
+        return out.cpu()
+
+    plain, out = _with_specials(cache, specials, contexts, blocks, offsets, device, run)
+    _assert_same(out, _expect(plain, specials, lambda item, key: [item], group))
+
+
+@pytest.mark.parametrize("dim", [32, 64, 256])
+def test_a_cache_of_nans_gives_nans(device, dim):
+    """V all NaN in one item's pages, decode and prefill; the others' rows stay."""
+    g = torch.Generator().manual_seed(dim)
+    queries, contexts = [70, 33], [300, 90]
+    cache, k, v, blocks, offsets = _setup(g, contexts, 2, dim, torch.bfloat16, False, device,
+                                          "token_major")
+    q = torch.randn(sum(queries), 8, dim, generator=g).to(torch.bfloat16)
+    args = (device, q, cache, k, v, blocks, offsets, queries, contexts, dim)
+    plain = _prefill(*args)[0]
+    for b in blocks[:offsets[1]].tolist():
+        cache.value[0][16 * b:16 * b + 16] = NAN
+    out = _prefill(*args)[0]
+    assert bool(out[:70].isnan().all()) and torch.equal(out[70:], plain[70:])

@@ -350,66 +350,69 @@ __device__ __forceinline__ void store_row(T* o, const float (&x)[N], float inv, 
     }
 }
 
-// One row by one wave in plain fp32 over keys [k_begin, k_end): the answer for
-// a row whose accumulators end non-finite. An infinity in V meets zero terms
-// above (the remainder of an exact P, masked or repeated keys), and 0 * inf is
-// NaN where the sum over the row's own keys may be infinite. Lane l scores
-// key l of each 64, and holds the output dims l, l + 64, ...
-template <typename T, bool F8, int D>
-__device__ __forceinline__ void exact_row(const GeneralAttention& a, const T* q,
-                                                    int kvh, int64_t table, int64_t k_begin,
-                                                    int64_t k_end, float& m, float& l,
-                                                    float (&acc)[(D + 63) / 64]) {
-    constexpr int DI = (D + 63) / 64;
-    const int lane = threadIdx.x & 63;
-    const float qscale = a.scale * kLog2eG * a.k_scale;
-    m = -INFINITY;
-    l = 0.f;
-#pragma unroll
-    for (int i = 0; i < DI; ++i) acc[i] = 0.f;
-    for (int64_t t0 = k_begin; t0 < k_end; t0 += 64) {
-        const int64_t t = min(t0 + lane, k_end - 1);
-        const int64_t page = t / a.block_size;
-        const int64_t base = (a.blocks[table + page] * a.block_size + (t - page * a.block_size)) *
-                                 a.css + int64_t(kvh) * a.chs;
-        float s = 0.f;
-        for (int d = 0; d < D; d += 8) {
-            float x[8];
-            load8<T, F8, true>(a.k, base + d, 8, x);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s = fmaf(to_f<T>(q[d + i]) * qscale, x[i], s);
-        }
-        if (t0 + lane >= k_end) s = -INFINITY;
-        const float mn = fmaxf(m, wave_max(s));
-        const float ref = mn == -INFINITY ? 0.f : mn;
-        const float alpha = exp2f(m - ref);
-        const float p = exp2f(s - ref);
-        l = l * alpha + wave_sum(p);
-        m = mn;
-#pragma unroll
-        for (int i = 0; i < DI; ++i) acc[i] *= alpha;
-        const int n = int(min<int64_t>(64, k_end - t0));
-        for (int j = 0; j < n; ++j) {
-            const float pj = __shfl(p, j, 64);
-            const int64_t row = int64_t(uint64_t(uint32_t(__shfl(int(uint64_t(base) >> 32), j, 64)))
-                                            << 32 |
-                                        uint32_t(__shfl(int(uint32_t(base)), j, 64)));
-#pragma unroll
-            for (int i = 0; i < DI; ++i) {
-                const int d = lane + 64 * i;
-                if (d < D) acc[i] = fmaf(pj, load1<T, F8>(a.v, row + d), acc[i]);
-            }
-        }
-    }
+// V with infinities or NaNs. They meet zero weights above - masked and repeated
+// keys, the remainder of an exact P - and 0 * inf is NaN where the sum over a
+// row's own keys may be an infinity, or finite. So a workgroup whose
+// accumulators end non-finite goes through its keys once more, EXACT: such
+// elements enter P.V as 0, for each output dim the first key with a positive
+// and with a negative one is noted (NaNs count as both), and the rows that see
+// that key take the infinity, or the two as a NaN. Other rows keep their bits.
+// In us, calls with one infinity against the same in fp32 on the vector units:
+// 64 x 2048 decode rows, heads of 64 165 -> 70; 4 x 512 queries over 2048 tokens,
+// heads of 64 / 256 2241 / 3298 -> 191 / 440; with NaNs throughout, 16 x 2048
+// decode rows, heads of 64 / 256 54 / 87 -> 54 / 268. (The second pass called out
+// of line cost every call scratch memory, 5 us and more.)
+
+template <typename T>
+__device__ __forceinline__ bool non_finite(uint32_t h) {  // of the low 16 bits
+    constexpr uint32_t kExp = std::is_same_v<T, __bf16> ? 0x7f80u : 0x7c00u;
+    return (h & kExp) == kExp;
 }
 
-template <int N>
-__device__ __forceinline__ bool all_finite(const float (&x)[N], float den) {
-    bool ok = den < INFINITY;  // false for NaN too
-#pragma unroll
-    for (int i = 0; i < N; ++i) ok = ok && fabsf(x[i]) < INFINITY;
-    return ok;
+// Zeroes the non-finite ones of a word's two elements: those whose magnitude,
+// as an integer, exceeds the largest finite one's. Returns 0xffff in their halves.
+template <typename T>
+__device__ __forceinline__ uint32_t drop_non_finite(uint32_t& w) {
+    typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+    constexpr int16_t kMax = std::is_same_v<T, __bf16> ? 0x7f7f : 0x7bff;
+    const i16x2 over = (i16x2{kMax, kMax} - __builtin_bit_cast(i16x2, w & 0x7fff7fffu)) >> 15;
+    const uint32_t mask = __builtin_bit_cast(uint32_t, over);
+    w &= ~mask;
+    return mask;
 }
+
+// The same for the NaNs (0x7f, 0xff) of four FP8 elements; a bit for any.
+__device__ __forceinline__ uint32_t drop_fp8_nan(uint32_t& w) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (((w >> (8 * i)) & 0x7f) == 0x7f) {
+            w &= ~(0xffu << (8 * i));
+            any = 1;
+        }
+    return any;
+}
+
+template <int D>
+struct FirstSpecial {
+    int plus[D], minus[D];  // key index, by output dim
+    __device__ __forceinline__ void clear(int thread, int threads) {
+        for (int i = thread; i < D; i += threads) plus[i] = minus[i] = INT32_MAX;
+    }
+    // Notes element h of `dim` at `key` if it is not finite.
+    template <typename T>
+    __device__ __forceinline__ void note(uint32_t h, int dim, int key) {
+        constexpr uint32_t kMant = std::is_same_v<T, __bf16> ? 0x7fu : 0x3ffu;
+        if (!non_finite<T>(h)) return;
+        const bool nan = (h & kMant) != 0, neg = (h & 0x8000u) != 0;
+        if (nan || !neg) atomicMin(&plus[dim], key);
+        if (nan || neg) atomicMin(&minus[dim], key);
+    }
+    // What a row that sees keys below `bound` adds to its sum.
+    __device__ __forceinline__ float value(int dim, int64_t bound) const {
+        return (plus[dim] < bound ? INFINITY : 0.f) + (minus[dim] < bound ? -INFINITY : 0.f);
+    }
+};
 
 // Few query rows against many keys: decode, and prefill calls of a few
 // queries. A workgroup serves up to 16 (query token, query head) rows of one
@@ -442,6 +445,8 @@ rows_attention_kernel(GeneralAttention a) {
     constexpr int VW = VE / 2;           // V words per key, widened
     __shared__ float part_acc[(NW - 1) * VE * 4 * 64];
     __shared__ float part_ml[NW - 1][2][64];
+    __shared__ FirstSpecial<D> special;
+    __shared__ bool again[NW];
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int col = lane & 15, quad = lane >> 4;
@@ -585,9 +590,91 @@ rows_attention_kernel(GeneralAttention a) {
     };
 
     gf32x4 acc[VE];  // acc[e][v]: dim VE * (4 * quad + v) + e of the lane's row
+    float m = -INFINITY, l = 0.f;
 #pragma unroll
     for (int e = 0; e < VE; ++e) acc[e] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
+    float x[4 * NT];
+    auto scores = [&](int64_t t0) {
+        // Keys of the chunk from this quad's first on that the row sees.
+        const int left = int(max<int64_t>(min<int64_t>(bound - t0, CH), 0)) - 4 * quad;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            gf32x4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                if constexpr (F8) sc = mfma32<T>(fp8x8_widen<T>(kreg[j][s]), qb[s], sc);
+                else sc = mfma32<T>(kreg[j][s], qb[s], sc);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                x[4 * j + i] = 16 * j + i < left ? sc[i] * qscale : -INFINITY;
+        }
+    };
+    auto attend = [&]<bool EXACT>(std::bool_constant<EXACT>, int64_t t0, int64_t off) {
+        float alpha;
+        if (softmax_step<T>(x, m, l, alpha)) {
+#pragma unroll
+            for (int e = 0; e < VE; ++e) acc[e] *= alpha;
+        }
+        if constexpr (EXACT) {
+            static_assert(NT == 2, "one group of 32 keys");
+            uint32_t flagged = 0;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    uint32_t any = 0;
+#pragma unroll
+                    for (int w = 0; w < (VB + 3) / 4; ++w) {
+                        if constexpr (F8) any |= drop_fp8_nan(vreg[j][i][w]);
+                        else any |= drop_non_finite<T>(vreg[j][i][w]);
+                    }
+                    flagged |= uint32_t(any != 0) << (4 * j + i);
+                }
+#pragma unroll 1
+            for (int e = 0; e < 8; ++e) {
+                const bool mine = (flagged >> e) & 1;
+                if (!__any(mine)) continue;
+                const int key = 16 * (e / 4) + 4 * quad + e % 4;
+                const char* const vk = vc + at(off, key) + col * VB;
+                if (!mine || t0 + key >= k_end) continue;
+#pragma unroll 1
+                for (int n = 0; n < VE; ++n) {
+                    uint32_t h;
+                    if constexpr (F8) {
+                        const uint32_t x = reinterpret_cast<const uint8_t*>(vk)[n];
+                        h = (x & 0x7f) == 0x7f ? 0x7fffu : 0u;
+                    } else {
+                        h = reinterpret_cast<const uint16_t*>(vk)[n];
+                    }
+                    special.template note<T>(h, VE * col + n, int(t0) + key);
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < NT / 2; ++g) {
+            float p[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[i] = x[8 * g + i];
+            U16x8 hi, lo;
+            split_p<T>(p, hi, lo);
+#pragma unroll
+            for (int w = 0; w < VW; ++w) {
+                U16x8 even, odd;
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    const int j = 2 * g + y / 2, i = 2 * (y & 1);
+                    const uint32_t v0 = v_word(j, i, w), v1 = v_word(j, i + 1, w);
+                    even.w[y] = pair_lo(v0, v1);
+                    odd.w[y] = pair_hi(v0, v1);
+                }
+                acc[2 * w] = mfma32<T>(even, hi, acc[2 * w]);
+                acc[2 * w + 1] = mfma32<T>(odd, hi, acc[2 * w + 1]);
+                acc[2 * w] = mfma32<T>(even, lo, acc[2 * w]);
+                acc[2 * w + 1] = mfma32<T>(odd, lo, acc[2 * w + 1]);
+            }
+        }
+    };
 
     // Wave w takes chunks w, w + NW, ... of the keys.
     int64_t t0 = k_begin + int64_t(wave) * CH;
@@ -601,53 +688,12 @@ rows_attention_kernel(GeneralAttention a) {
         for (; t0 < k_end; t0 += kStep) {
             off = resolve(t0 + kStep, id);
             id = load_id(t0 + 2 * kStep);
-            float x[4 * NT];
-            // Keys of the chunk from this quad's first on that the row sees.
-            const int left = int(max<int64_t>(min<int64_t>(bound - t0, CH), 0)) - 4 * quad;
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                gf32x4 sc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    if constexpr (F8) sc = mfma32<T>(fp8x8_widen<T>(kreg[j][s]), qb[s], sc);
-                    else sc = mfma32<T>(kreg[j][s], qb[s], sc);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    x[4 * j + i] = 16 * j + i < left ? sc[i] * qscale : -INFINITY;
-            }
+            scores(t0);
             load_k(off);
             // The scheduler would gather V's operands ahead of these loads,
             // and wait for V there.
             __builtin_amdgcn_sched_barrier(0);
-            float alpha;
-            if (softmax_step<T>(x, m, l, alpha)) {
-#pragma unroll
-                for (int e = 0; e < VE; ++e) acc[e] *= alpha;
-            }
-#pragma unroll
-            for (int g = 0; g < NT / 2; ++g) {
-                float p[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) p[i] = x[8 * g + i];
-                U16x8 hi, lo;
-                split_p<T>(p, hi, lo);
-#pragma unroll
-                for (int w = 0; w < VW; ++w) {
-                    U16x8 even, odd;
-#pragma unroll
-                    for (int y = 0; y < 4; ++y) {
-                        const int j = 2 * g + y / 2, i = 2 * (y & 1);
-                        const uint32_t v0 = v_word(j, i, w), v1 = v_word(j, i + 1, w);
-                        even.w[y] = pair_lo(v0, v1);
-                        odd.w[y] = pair_hi(v0, v1);
-                    }
-                    acc[2 * w] = mfma32<T>(even, hi, acc[2 * w]);
-                    acc[2 * w + 1] = mfma32<T>(odd, hi, acc[2 * w + 1]);
-                    acc[2 * w] = mfma32<T>(even, lo, acc[2 * w]);
-                    acc[2 * w + 1] = mfma32<T>(odd, lo, acc[2 * w + 1]);
-                }
-            }
+            attend(std::false_type{}, t0, off);
             load_v(off);
             // Nothing is written; but a possible write keeps the compiler from
             // turning the loaded values carried into the next iteration into
@@ -660,7 +706,8 @@ rows_attention_kernel(GeneralAttention a) {
     // Merge the waves' partial results: out = sum_w 2^(m_w - M) acc_w /
     // sum_w 2^(m_w - M) l_w per row (M the largest m_w); a row with no key
     // in any wave gives zeros.
-    if (wave > 0) {
+    auto publish = [&] {
+        if (wave == 0) return;
 #pragma unroll
         for (int e = 0; e < VE; ++e)
 #pragma unroll
@@ -668,8 +715,40 @@ rows_attention_kernel(GeneralAttention a) {
                 part_acc[((wave - 1) * VE * 4 + 4 * e + v) * 64 + lane] = acc[e][v];
         part_ml[wave - 1][0][lane] = m;
         part_ml[wave - 1][1][lane] = l;
-    }
+    };
+    publish();
+    gf32x4 sums = acc[0];  // four chains
+#pragma unroll
+    for (int e = 1; e < VE; ++e) sums += acc[e];
+    const float sum = l + ((sums[0] + sums[1]) + (sums[2] + sums[3]));
+    const bool bad = __any(col < nrows && !(fabsf(sum) < INFINITY));
+    if (lane == 0) again[wave] = bad;
     __syncthreads();
+    // Unlikely, said so to have what follows it next in line.
+    if (__builtin_expect(again[0] || again[1] || again[2] || again[3], 0)) {  // uniform
+#pragma unroll
+        for (int e = 0; e < VE; ++e) acc[e] = gf32x4{0.f, 0.f, 0.f, 0.f};
+        m = -INFINITY;
+        l = 0.f;
+        special.clear(threadIdx.x, 64 * NW);
+        __syncthreads();
+        for (int64_t t = k_begin + int64_t(wave) * CH; t < k_end; t += NW * CH) {
+            const int64_t off = resolve(t, load_id(t));
+            load_k(off);
+            scores(t);
+            load_v(off);
+            attend(std::true_type{}, t, off);
+        }
+        l = quad_sum(l);
+        publish();
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int e = 0; e < VE; ++e)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[e][v] += special.value(VE * (4 * quad + v) + e, bound);
+        }
+    }
     if (wave > 0) return;
     float mx = m;
 #pragma unroll
@@ -693,28 +772,7 @@ rows_attention_kernel(GeneralAttention a) {
     for (int v = 0; v < 4; ++v)
 #pragma unroll
         for (int e = 0; e < VE; ++e) o[v * VE + e] = acc[e][v];
-    const uint64_t bad = __ballot(col < nrows && !all_finite(o, den));
-    for (int r = 0; bad != 0 && r < nrows; ++r) {
-        if ((bad & (0x0001000100010001ull << r)) == 0) continue;
-        const int64_t tr = tok0 + r / hw;
-        const int hr = kvh * group + g0 + r % hw;
-        float em, el, eacc[(D + 63) / 64];
-        exact_row<T, F8, D>(a, static_cast<const T*>(a.q) + tr * a.qts + hr * a.qhs, kvh, table,
-                            k_begin, min(first_end + r / hw, k_end), em, el, eacc);
-        const int64_t pr = (item * a.heads + hr) * a.splits + split;
-#pragma unroll
-        for (int i = 0; i < (D + 63) / 64; ++i) {
-            const int d = lane + 64 * i;
-            if (d >= D) continue;
-            if (a.splits > 1) a.part_o[pr * D + d] = eacc[i];
-            else out[tr * a.ots + hr * a.ohs + d] = static_cast<T>(eacc[i] * (a.v_scale / el));
-        }
-        if (a.splits > 1 && lane == 0) {
-            a.part_ml[2 * pr] = em;
-            a.part_ml[2 * pr + 1] = el;
-        }
-    }
-    if (col >= nrows || (bad >> col & 0x0001000100010001ull) != 0) return;
+    if (col >= nrows) return;
     if (a.splits > 1) {  // the split's partials, merged by general_merge
         float* const po = a.part_o + part * D + 4 * VE * quad;
 #pragma unroll
@@ -761,13 +819,15 @@ tiles_attention_kernel(GeneralAttention a) {
     constexpr int kBuf = KC * KSTR + D * VSTR;
     __shared__ __align__(16) unsigned char smem_all[HV * 2 * kBuf];
     __shared__ int64_t row_offs[HV][2][KC];  // byte offsets of a chunk's cache rows
-    const int half = HV == 1 ? 0 : threadIdx.x / NT;
-    const int tid = threadIdx.x % NT;  // within the half
+    __shared__ FirstSpecial<D> special;
+    __shared__ bool again[HV * kRowWaves];
+    // (Uniform per wave, said so to keep them in scalar registers.)
+    const int half = HV == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    int tid = threadIdx.x % NT;  // within the half
     unsigned char* const smem = smem_all + half * 2 * kBuf;
     int64_t (*const row_off)[KC] = row_offs[half];
-    const int wave = tid >> 6;
-    const int lane = tid & 63;
-    const int col = lane & 15, quad = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int lane = tid & 63, col = lane & 15, quad = lane >> 4;
 
     const int group = a.heads / a.kv_heads;
     const int kvh = int(blockIdx.x % a.kv_heads);
@@ -808,13 +868,6 @@ tiles_attention_kernel(GeneralAttention a) {
 
     gf32x4 acc[RT][DT];  // acc[t][d][v]: dim 16 * d + 4 * quad + v of row 16 * t + col
     float m[RT], l[RT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        m[t] = -INFINITY;
-        l[t] = 0.f;
-#pragma unroll
-        for (int d = 0; d < DT; ++d) acc[t][d] = gf32x4{0.f, 0.f, 0.f, 0.f};
-    }
 
     // Staging. K: 8-element pieces, a key's pieces side by side in the lanes.
     // V: 4 keys x 8 dims per task, transposed in registers; 8 lanes hold 64
@@ -903,58 +956,57 @@ tiles_attention_kernel(GeneralAttention a) {
         }
     };
 
-    int64_t id = 0;
     constexpr int kStep = HV * KC;
     const int64_t first = half * KC;
-    if (kv_max > 0) {  // uniform per workgroup
-        put_offset(first, load_id(first), 0);
-        id = load_id(first + kStep);
-        __syncthreads();
-        load_stage(0);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        m[t] = -INFINITY;
+        l[t] = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) acc[t][d] = gf32x4{0.f, 0.f, 0.f, 0.f};
     }
-    asm volatile("" ::: "memory");  // keeps carried loads where they are issued
-    int cur = 0;
-    for (int64_t step = 0; step < kv_max; step += kStep, cur ^= 1) {
-        const int64_t t0 = step + first;  // this half's chunk
-        unsigned char* const buf = smem + cur * kBuf;
-        store_stage(buf);
-        put_offset(t0 + kStep, id, cur ^ 1);
-        // After it, every wave is also past the reads of what the next
-        // iteration overwrites (the other buffer, these offsets' predecessors).
-        __syncthreads();
-        id = load_id(t0 + 2 * kStep);
-        load_stage(cur ^ 1);
-        if (t0 >= wave_end) continue;
+    auto attend = [&]<bool EXACT>(std::bool_constant<EXACT>, int64_t t0,
+                                  const unsigned char* buf) {
         const unsigned char* const ks = buf + col * KSTR + quad * 16;
         const unsigned char* const vs = buf + KC * KSTR + col * VSTR + quad * 16;
         // Operands are read ahead of the MFMAs that take them, all of K's at
         // once and V's behind Q.K^T: the compiler's own order reads one or two
         // ahead and waits out the LDS latency 32 times per chunk.
-        U16x8 kk[2 * G][KS];
+        auto k_at = [&](int j, int s) {
+            return *reinterpret_cast<const U16x8*>(ks + 16 * j * KSTR + 64 * s);
+        };
+        auto v_at = [&](int d, int g) {
+            return *reinterpret_cast<const U16x8*>(vs + 16 * d * VSTR + 64 * g);
+        };
+        U16x8 kk[2 * G][KS], vv[DT][G];  // (exact: read where they are taken)
+        if constexpr (!EXACT) {
 #pragma unroll
-        for (int j = 0; j < 2 * G; ++j)
+            for (int j = 0; j < 2 * G; ++j)
 #pragma unroll
-            for (int s = 0; s < KS; ++s)
-                kk[j][s] = *reinterpret_cast<const U16x8*>(ks + 16 * j * KSTR + 64 * s);
-        __builtin_amdgcn_sched_barrier(0);
+                for (int s = 0; s < KS; ++s) kk[j][s] = k_at(j, s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         gf32x4 sc[RT][2 * G];
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
             for (int j = 0; j < 2 * G; ++j) sc[t][j] = gf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 2 * G; ++j)
+        for (int j = 0; j < 2 * G; ++j) {
+            if constexpr (EXACT) asm volatile("" ::: "memory");  // a few registers at a time
 #pragma unroll
             for (int s = 0; s < KS; ++s)
 #pragma unroll
-                for (int t = 0; t < RT; ++t) sc[t][j] = mfma32<T>(kk[j][s], qb[t][s], sc[t][j]);
-        U16x8 vv[DT][G];
+                for (int t = 0; t < RT; ++t)
+                    sc[t][j] = mfma32<T>(EXACT ? k_at(j, s) : kk[j][s], qb[t][s], sc[t][j]);
+        }
+        if constexpr (!EXACT) {
 #pragma unroll
-        for (int d = 0; d < DT; ++d)
+            for (int d = 0; d < DT; ++d)
 #pragma unroll
-            for (int g = 0; g < G; ++g)
-                vv[d][g] = *reinterpret_cast<const U16x8*>(vs + 16 * d * VSTR + 64 * g);
-        __builtin_amdgcn_sched_barrier(0);
+                for (int g = 0; g < G; ++g) vv[d][g] = v_at(d, g);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         U16x8 hi[RT][G], lo[RT][G];
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -978,21 +1030,115 @@ tiles_attention_kernel(GeneralAttention a) {
                 split_p<T>(p, hi[t][g], lo[t][g]);
             }
         }
+        [[maybe_unused]] uint32_t flagged[G] = {};  // by tile of the output dims
 #pragma unroll
         for (int d = 0; d < DT; ++d)
 #pragma unroll
-            for (int g = 0; g < G; ++g)
+            for (int g = 0; g < G; ++g) {
+                if constexpr (EXACT) {
+                    asm volatile("" ::: "memory");
+                    vv[d][g] = v_at(d, g);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        if (drop_non_finite<T>(vv[d][g].w[w])) flagged[g] |= 1u << d;
+                }
 #pragma unroll
                 for (int t = 0; t < RT; ++t) {
                     acc[t][d] = mfma32<T>(vv[d][g], hi[t][g], acc[t][d]);
                     acc[t][d] = mfma32<T>(vv[d][g], lo[t][g], acc[t][d]);
                 }
-    }
+            }
+        if constexpr (EXACT) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll 1
+                for (int d = 0; d < DT; ++d) {
+                    if (!((flagged[g] >> d) & 1)) continue;
+#pragma unroll 1
+                    for (int e = 0; e < 8; ++e) {
+                        const int key = int(t0) + 32 * g + 16 * (e / 4) + 4 * quad + e % 4;
+                        const uint32_t h = *reinterpret_cast<const uint16_t*>(
+                            vs + 16 * d * VSTR + 64 * g + 2 * e);
+                        if (key < kv_max) special.template note<T>(h, 16 * d + col, key);
+                    }
+                }
+        }
+    };
 
+    int64_t id = 0;
+    if (kv_max > 0) {  // uniform per workgroup
+        put_offset(first, load_id(first), 0);
+        id = load_id(first + kStep);
+        __syncthreads();
+        load_stage(0);
+    }
+    asm volatile("" ::: "memory");  // keeps carried loads where they are issued
+    int cur = 0;
+    for (int64_t step = 0; step < kv_max; step += kStep, cur ^= 1) {
+        const int64_t t0 = step + first;  // this half's chunk
+        unsigned char* const buf = smem + cur * kBuf;
+        store_stage(buf);
+        put_offset(t0 + kStep, id, cur ^ 1);
+        // After it, every wave is also past the reads of what the next
+        // iteration overwrites (the other buffer, these offsets' predecessors).
+        __syncthreads();
+        id = load_id(t0 + 2 * kStep);
+        load_stage(cur ^ 1);
+        if (t0 < wave_end) attend(std::false_type{}, t0, buf);
+    }
+    // The lane's place once more, from the hardware: not kept through the loop.
+    lane = int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    asm volatile("" : "+v"(lane));
+    col = lane & 15;
+    quad = lane >> 4;
+    tid = 64 * wave + lane;
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        gf32x4 sums = acc[t][0];  // four chains
+#pragma unroll
+        for (int d = 1; d < DT; ++d) sums += acc[t][d];
+        const float sum = l[t] + ((sums[0] + sums[1]) + (sums[2] + sums[3]));
+        bad = bad || (wr0 + 16 * t + col < total && !(fabsf(sum) < INFINITY));
+    }
+    bad = __any(bad);
+    if (lane == 0) again[half * kRowWaves + wave] = bad;
+    __syncthreads();  // also: every wave is past its reads of the buffers
+    bad = false;
+#pragma unroll
+    for (int w = 0; w < HV * kRowWaves; ++w) bad = bad || again[w];
+    if (__builtin_expect(bad, 0)) {  // uniform
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            m[t] = -INFINITY;
+            l[t] = 0.f;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) acc[t][d] = gf32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        special.clear(threadIdx.x, HV * NT);
+        for (int64_t step = 0; step < kv_max; step += kStep) {
+            const int64_t t0 = step + first;
+            put_offset(t0, load_id(t0), 0);
+            __syncthreads();
+            load_stage(0);
+            store_stage(smem);
+            __syncthreads();
+            if (t0 < wave_end) attend(std::true_type{}, t0, smem);
+            __syncthreads();  // every wave is past its reads of both
+        }
+        if (half == 0) {  // once, where the halves merge
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[t][d][v] += special.value(16 * d + 4 * quad + v, bound[t]);
+        }
+    }
     if constexpr (HV > 1) {
         // The second half's (max, sum, accumulators) join the first's, lane by
         // lane, through the staging buffers.
-        __syncthreads();  // every wave is past its reads of them
         float* const part = reinterpret_cast<float*>(smem_all) + wave * 64 + lane;
         constexpr int kStride = 64 * kRowWaves;
         static_assert((RT * (4 * DT + 2)) * kStride * 4 <= HV * 2 * kBuf, "merge fits the buffers");
@@ -1029,28 +1175,7 @@ tiles_attention_kernel(GeneralAttention a) {
         const float den = quad_sum(l[t]);
         const float inv = den > 0.f ? a.v_scale / den : 0.f;
         const int64_t r = wr0 + 16 * t + col;
-        bool ok = den < INFINITY;  // false for NaN too
-#pragma unroll
-        for (int d = 0; d < DT; ++d)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) ok = ok && fabsf(acc[t][d][v]) < INFINITY;
-        const uint64_t bad = __ballot(r < total && !ok);
-        for (int c = 0; bad != 0 && c < 16; ++c) {
-            if ((bad & (0x0001000100010001ull << c)) == 0) continue;
-            const int64_t rc = wr0 + 16 * t + c, qc = rc / group;
-            const int hc = kvh * group + int(rc % group);
-            float em, el, eacc[(D + 63) / 64];
-            exact_row<T, F8, D>(a, static_cast<const T*>(a.q) + (tok0 + qc) * a.qts + hc * a.qhs,
-                                kvh, table, 0, before + qc + 1, em, el, eacc);
-#pragma unroll
-            for (int i = 0; i < (D + 63) / 64; ++i) {
-                const int d = lane + 64 * i;
-                if (d < D)
-                    out[(tok0 + qc) * a.ots + hc * a.ohs + d] =
-                        static_cast<T>(eacc[i] * (a.v_scale / el));
-            }
-        }
-        if (r >= total || (bad >> col & 0x0001000100010001ull) != 0) continue;
+        if (r >= total) continue;
         T* const o = out + (tok0 + r / group) * a.ots +
                      (kvh * group + int(r % group)) * a.ohs + 4 * quad;
 #pragma unroll
