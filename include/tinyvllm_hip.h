@@ -358,7 +358,8 @@ int tvllm_argmax(const void* logits, int64_t rows, int64_t vocab,
  * temperature > 0 samples; temperature 0 rows take the argmax.
  * workspace (optional, 16-byte aligned): with
  * tvllm_sample_split_workspace_size(rows, vocab) bytes every pass over a row
- * is spread over several workgroups (four launches); with
+ * is spread over several workgroups (four launches; one, a workgroup per row,
+ * where a row has at most 8192 tokens); with
  * tvllm_sample_workspace_size(rows, vocab) bytes only the search for the
  * row's maximum is (two launches); with workspace_bytes 0 each row's
  * workgroup draws alone. Same result in all three.

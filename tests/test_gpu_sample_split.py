@@ -7,7 +7,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-PARAMS = [(t, k, p) for t in (0.0, 0.05, 0.7, 1.0, 30.0) for k in (0, 1, 3, 40, 5000)
+PARAMS = [(t, k, p) for t in (0.0, 0.05, 0.7, 1.0, 30.0, float("inf"))
+          for k in (0, 1, 3, 40, 4096, 4097, 5000)
           for p in (1.0, 0.9, 0.5, 1e-6)]
 
 
