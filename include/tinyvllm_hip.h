@@ -399,11 +399,10 @@ int tvllm_resolve_tokens(int64_t* tokens, const int64_t* src, const int64_t* pre
  * with 16-byte aligned cache rows on MFMAs (workgroups of 64 or 128 (query
  * token, query head) rows of one item and KV head, or of up to 16 where an
  * item has at most 32), others in fp32 (up to 16 rows).
- * workspace: >= tvllm_paged_prefill_workspace_size(dtype, cache_dtype)
- * bytes, 4-byte aligned; left as it is. (A bf16 cache's V is converted to
- * fp16 for the P.V products; a workgroup in which a V value of 65536 or more
- * in magnitude, an infinity or a NaN enters a product redoes its queries
- * exactly. The flag that once asked for that lived in the workspace.)
+ * workspace, workspace_bytes: not used (null and 0 will do). A bf16 cache's V
+ * is converted to fp16 for the P.V products at head_dim 128; a workgroup in
+ * which a V value of 65536 or more in magnitude, an infinity or a NaN enters a
+ * product redoes its queries exactly.
  * Replaces: CudaAttention._attend's per-row gather + SDPA for rows with
  * history (reference tinyvllm/runtime/attention.py:102-151, 235-285). */
 int tvllm_paged_prefill(const void* q, int64_t q_token_stride,
@@ -421,9 +420,8 @@ int tvllm_paged_prefill(const void* q, int64_t q_token_stride,
                         int dtype, int cache_dtype, float k_scale,
                         float v_scale, tvllm_stream_t stream);
 
-/* Bytes of workspace tvllm_paged_prefill asks for: 8 for a bf16 query and
- * cache, 0 otherwise. No counterpart in the reference
- * (its prefill path allocates nothing of the kind). */
+/* Bytes of workspace tvllm_paged_prefill asks for: 0. No counterpart in the
+ * reference (its prefill path allocates nothing of the kind). */
 int64_t tvllm_paged_prefill_workspace_size(int dtype, int cache_dtype);
 
 #ifdef __cplusplus

@@ -251,15 +251,14 @@ def test_prefill_chunks_with_history(device, heads, kv_heads, items, bs, layout)
 
 def test_prefill_v_beyond_fp16_range_takes_the_exact_path(device):
     """P.V runs on fp16 MFMAs with V converted from bf16; V values of 65536
-    or more (or inf/NaN) reach the outputs as fp16 infinities, and a wave
-    whose accumulators end non-finite makes the call recompute on bf16
-    MFMAs. Every case matches the oracle (a missed recompute would leave
-    infinities or NaNs in the output), and the fallback guard is back to
-    zero after each. 65280 is the largest bf16 below 65536 (exact in fp16);
+    or more (or inf/NaN) reach the outputs as fp16 infinities, and a
+    workgroup with a wave whose accumulators end non-finite redoes its
+    queries on bf16 MFMAs. Every case matches the oracle (a missed recompute
+    would leave infinities or NaNs in the output), and the other item keeps
+    its bits. 65280 is the largest bf16 below 65536 (exact in fp16);
     65536 is the smallest that overflows; a value in the last pages is seen
     only by the chunk's last queries."""
     from helpers import assert_within_ulp
-    from tinyvllm.kernels import paged_prefill as PP
     from tinyvllm.kernels.paged_prefill import paged_prefill_attention
     from tinyvllm.runtime.contracts import MultiQueryMetadata
 
@@ -282,6 +281,7 @@ def test_prefill_v_beyond_fp16_range_takes_the_exact_path(device):
     late_row = torch.tensor([blocks[boff[1] - 1] * bs + (700 - 1) % bs])  # key 699
     for case in ("large", "none", "65536_late", "65280", "-65536_first"):
         v = torch.randn(pool * bs, kv_heads, d, generator=g)
+        plain = v.clone()
         if case == "large":  # a few values fp16 cannot hold, in the first item's pages
             v[first_rows, 2, 7] = 3.0e5
             v[first_rows[:1], 5, 100] = -70000.0
@@ -301,8 +301,12 @@ def test_prefill_v_beyond_fp16_range_takes_the_exact_path(device):
         torch.cuda.synchronize()
         print(f"prefill V case {case}", flush=True)
         assert_within_ulp(out.cpu(), expect, ulps=2.0)
-        guard = PP._GUARDS[(out.device, torch.cuda.current_stream(out.device).cuda_stream)]
-        assert int(guard.count_nonzero()) == 0
+        # Item 1's workgroups have their own pages: the same bits as without
+        # item 0's large values.
+        cache = _Cache(k.to(device), plain.to(torch.bfloat16).to(device), bs)
+        without = torch.zeros(q.shape, dtype=q.dtype, device=device)
+        paged_prefill_attention(q.to(device), cache, 0, meta, without, scale=d ** -0.5)
+        assert torch.equal(out[qoff[1]:], without[qoff[1]:])
 
 
 # ----------------------------------------------------------------- pointwise --

@@ -271,9 +271,9 @@ def test_cache_layouts_give_bit_identical_runs(device, kv_dtype):
 
 def test_prefill_graphs_exact_fallback_for_v_beyond_fp16(device, monkeypatch):
     """A cache holding V values beyond the fp16 range (layer 0's V rows of
-    the packed projection scaled by 4e4): the prefill graphs' replays take
-    the exact bf16 fallback launch like eager prefill does, give the eager
-    logits and tokens, and leave the graphs' own fallback guard clear."""
+    the packed projection scaled by 4e4): the prefill graphs' replays redo the
+    queries exactly like eager prefill does, and give the eager logits and
+    tokens."""
     from tinyvllm.executor import Executor
     from tinyvllm.runtime.prefill_graphs import PrefillGraphs
 
@@ -314,9 +314,6 @@ def test_prefill_graphs_exact_fallback_for_v_beyond_fp16(device, monkeypatch):
         torch.cuda.synchronize()
         v0 = runner.kv_cache.value[0].float()  # slots never written hold NaN
         assert torch.nan_to_num(v0, nan=0.0).abs().max().item() >= 65536.0
-        if not eager:
-            guard = runner.prefill_graphs.guard
-            assert guard is not None and int(guard.count_nonzero()) == 0
         results[eager] = (logits, tokens)
         executor.clear()
     assert len(replays) == len(steps)

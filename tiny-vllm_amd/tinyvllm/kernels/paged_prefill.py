@@ -6,9 +6,6 @@ wrapper (runtime/prefill.py:15-225).
 """
 from __future__ import annotations
 
-import threading
-from contextlib import contextmanager
-
 import torch
 
 from tinyvllm.kernels._extension import (
@@ -53,8 +50,6 @@ def paged_prefill_attention(
     if items == 0 or m.max_query_len == 0:
         return
     cache_dtype, k_scale, v_scale = cache_format(cache)
-    guard = _guard(device, int(lib.tvllm_paged_prefill_workspace_size(
-        dtype_code(q.dtype), cache_dtype)))
     check(lib.tvllm_paged_prefill(
         q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), v.data_ptr(),
         output.data_ptr(), output.stride(0), output.stride(1),
@@ -62,51 +57,6 @@ def paged_prefill_attention(
         m.block_table_offsets.data_ptr(), m.context_lens.data_ptr(),
         items, m.max_query_len, q.shape[1], cache.num_kv_heads, q.shape[2],
         cache.num_slots, k.stride(0), k.stride(1), cache.block_size, float(scale),
-        None if guard is None else guard.data_ptr(), 0 if guard is None else guard.numel(),
-        dtype_code(q.dtype), cache_dtype, k_scale, v_scale, stream_of(device),
+        None, 0, dtype_code(q.dtype), cache_dtype, k_scale, v_scale, stream_of(device),
     ))
 
-
-_GUARDS: dict[tuple[torch.device, int], torch.Tensor] = {}
-_OWNED = threading.local()
-
-# Bytes of the workspace that a call passes along (the library's interface asks
-# for it; its kernels leave it as it is).
-GUARD_BYTES = 8
-
-
-@contextmanager
-def fallback_guard(guard: torch.Tensor):
-    """Calls inside this context use ``guard`` (zero-initialised uint8 of
-    GUARD_BYTES on the calls' device) as the workspace that the C entry asks
-    for (interface only: a workgroup whose V leaves fp16's range redoes its
-    own queries, and nothing is written there any more). A captured
-    graph owns its guard this way for the graph's lifetime, instead of one
-    keyed by the capture stream's handle, which torch may hand to another
-    stream once the capture stream is gone."""
-    if guard.dtype != torch.uint8 or guard.numel() < GUARD_BYTES or not guard.is_cuda:
-        raise ValueError(f"a fallback guard is a CUDA uint8 tensor of >= {GUARD_BYTES} bytes")
-    previous = getattr(_OWNED, "guard", None)
-    _OWNED.guard = guard
-    try:
-        yield guard
-    finally:
-        _OWNED.guard = previous
-
-
-def _guard(device: torch.device, nbytes: int) -> torch.Tensor | None:
-    """The zero-initialised fallback guard: the one ``fallback_guard``
-    installed, else that of ``device``'s current stream."""
-    if nbytes == 0:
-        return None
-    owned = getattr(_OWNED, "guard", None)
-    if owned is not None:
-        if owned.device != device or owned.numel() < nbytes:
-            raise RuntimeError("the installed fallback guard does not fit this call")
-        return owned
-    key = (device, stream_of(device))
-    guard = _GUARDS.get(key)
-    if guard is None or guard.numel() < nbytes:
-        guard = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-        _GUARDS[key] = guard
-    return guard

@@ -37,7 +37,6 @@ import torch
 
 from tinyvllm._validation import _check_positive_int
 from tinyvllm.batch import PreparedBatch
-from tinyvllm.kernels.paged_prefill import GUARD_BYTES, fallback_guard
 from tinyvllm.kernels.sampling import resolve_tokens, sample
 from tinyvllm.paged_kv import PagedKVCache
 from tinyvllm.runtime.attention import HipAttention
@@ -205,9 +204,6 @@ class PrefillGraphs:
         self.entries: dict[tuple[int, int], tuple[torch.cuda.CUDAGraph, torch.Tensor,
                                                   torch.Tensor]] = {}
         self.pool = None
-        # The prefill kernels' fallback guard of every captured graph: owned
-        # here, so it lives exactly as long as the graphs that point at it.
-        self.guard: torch.Tensor | None = None
 
     @torch.inference_mode()
     def capture(self, model: torch.nn.Module, inputs: PrefillInputs,
@@ -231,9 +227,8 @@ class PrefillGraphs:
         side = torch.cuda.Stream(device=inputs.device)
         side.wait_stream(self.stream)
         self.pool = torch.cuda.graph_pool_handle()
-        self.guard = torch.zeros(GUARD_BYTES, dtype=torch.uint8, device=inputs.device)
         try:
-            with torch.cuda.stream(side), fallback_guard(self.guard):
+            with torch.cuda.stream(side):
                 below = 0  # the previous token bucket
                 for tokens in TOKEN_BUCKETS:
                     if tokens > inputs.max_tokens:
@@ -292,4 +287,3 @@ class PrefillGraphs:
         self.stream.synchronize()
         self.entries.clear()
         self.pool = None
-        self.guard = None
