@@ -107,7 +107,8 @@ int tvllm_begin_decode(int64_t* table, int64_t table_size, const int64_t* update
  * copies in one launch. embed [vocab, width], cos and sin [max_position,
  * half], outputs [tokens, width] and [tokens, half], all dense and 16-byte
  * aligned, width and half multiples of 8. An id or position outside its
- * table gives a row of NaNs and reads nothing.
+ * table gives a row of NaNs and reads nothing; no later call refuses such a
+ * row (tvllm_sample answers token 0), so callers check their ids.
  * Replaces: nn.Embedding and RotaryEmbedding's gathers (reference
  *           tinyvllm/models/qwen3.py, layers.py:167-245). */
 int tvllm_embed_rope(const int64_t* ids, const int64_t* positions, int64_t tokens,
@@ -152,7 +153,7 @@ int64_t tvllm_paged_decode_split_plan(int64_t num_rows, int64_t num_heads,
  * alignment runs a workgroup of four waves per row, KV head and group of up
  * to 16 query heads, sharing each K/V load; when such units are few, each
  * row's keys split over several workgroups and a second launch merges their
- * partials. Head dims 32, 64, 128 and 256 with 16-byte aligned cache rows use
+ * partials. Head dims 32, 64, 128 and 256 with 16-byte aligned cache rows (8-byte ones of FP8) use
  * MFMAs there too (fp32 sums, weights as two 16-bit terms), others fp32
  * arithmetic on the vector units.
  * cache_dtype: dtype (caches hold q's element type; k_scale = v_scale = 1)
@@ -396,7 +397,7 @@ int tvllm_resolve_tokens(int64_t* tokens, const int64_t* src, const int64_t* pre
  * head_dim 128 runs the MFMA kernel (16-byte aligned Q and cache rows, cache
  * strides in whole 8-element units). Any other head_dim <= 256 runs the
  * kernels that tvllm_paged_decode has for the other shapes: 32, 64 and 256
- * with 16-byte aligned cache rows on MFMAs (workgroups of 64 or 128 (query
+ * with 16-byte aligned cache rows (8-byte ones of FP8) on MFMAs (workgroups of 64 or 128 (query
  * token, query head) rows of one item and KV head, or of up to 16 where an
  * item has at most 32), others in fp32 (up to 16 rows).
  * workspace, workspace_bytes: not used (null and 0 will do). A bf16 cache's V

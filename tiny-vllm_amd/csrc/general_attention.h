@@ -46,10 +46,10 @@ struct GeneralAttention {
 
 // Grid-level key splits of a decode launch of these kernels (1: none):
 // enough workgroups to fill the chip when there are few (row, KV head) units,
-// each split keeping at least two rounds of chunks for each of its waves.
+// each split keeping at least eight units of keys (split_unit).
 struct GeneralSplits {
     int64_t splits;  // workgroups per (row, KV head, head chunk)
-    int64_t keys;    // keys per split (a multiple of the kernel's chunk)
+    int64_t keys;    // keys per split (a multiple of the unit)
 };
 GeneralSplits general_decode_splits(int64_t rows, int64_t heads, int64_t kv_heads,
                                     int64_t head_dim, int64_t max_context);

@@ -30,7 +30,7 @@ namespace {
 constexpr int GH = 16;     // query heads per wave
 constexpr int DMAX = 256;  // largest head dim
 constexpr float kLog2eG = 1.4426950408889634f;
-constexpr int kRowWaves = 4;  // waves per workgroup of the row-tiled kernel
+constexpr int kRowWaves = 4;  // waves per workgroup of the matrix-core kernels (or half of one)
 
 // Eight elements of a cache row starting at element e (FP8: bytes), as
 // floats; elements at or past `left` read as 0.
@@ -1234,8 +1234,10 @@ general_merge(const float* __restrict__ part_o, const float* __restrict__ part_m
     }
 }
 
-// Keys per chunk of the row-tiled kernel at head dim D (LPK lanes per key).
-int64_t keys_per_chunk(int64_t D) { return D > 64 ? 64 / (D / 64) : 64; }
+// The unit of keys that decode splits are planned in: 64 up to head dim 64, 32
+// at 128, 16 at 256. Fixed, as callers size workspaces by the plan; the kernel's
+// own chunks are of 32 keys at every head dim.
+int64_t split_unit(int64_t D) { return D > 64 ? 64 / (D / 64) : 64; }
 
 bool rows_kernel_dim(int64_t D) { return D == 32 || D == 64 || D == 128 || D == 256; }
 
@@ -1247,19 +1249,21 @@ GeneralSplits general_decode_splits(int64_t rows, int64_t heads, int64_t kv_head
     if (rows <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || max_context <= 0 ||
         !rows_kernel_dim(head_dim))
         return p;
-    // Aim for 512 workgroups (two of four waves per CU); a split keeps at
-    // least two rounds of chunks per wave, and one merge lane per split.
+    // Aim for 512 workgroups (two of four waves per CU). A split keeps at
+    // least eight units: of the kernel's rounds (a 32-key chunk for each of
+    // four waves) four up to head dim 64, two at 128, one at 256, where it may
+    // also end inside a chunk. One merge lane per split.
     constexpr int64_t kTarget = 512, kMaxSplits = 64;
     const int64_t units = rows * kv_heads * ((heads / kv_heads + GH - 1) / GH);
-    const int64_t kpc = keys_per_chunk(head_dim);
-    const int64_t min_keys = 2 * kRowWaves * kpc;
+    const int64_t unit = split_unit(head_dim);
+    const int64_t min_keys = 8 * unit;
     int64_t s = std::min((kTarget + units - 1) / units, kMaxSplits);
     s = std::min(s, (max_context + min_keys - 1) / min_keys);
     if (s <= 1) return p;
     // Exactly s splits (a trailing one may hold no key: it writes an empty
     // partial), so the workspace never shrinks as max_context grows.
     p.splits = s;
-    p.keys = ((max_context + s - 1) / s + kpc - 1) / kpc * kpc;
+    p.keys = ((max_context + s - 1) / s + unit - 1) / unit * unit;
     return p;
 }
 
@@ -1289,8 +1293,9 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     const int64_t qpw = rows_kernel && group < GH ? GH / group : 1;
     g.q_vec = g.qts % 8 == 0 && g.qhs % 8 == 0 && aligned16(g.q);
     g.out_vec = g.ots % 4 == 0 && g.ohs % 4 == 0 && aligned8(g.out);
-    // Prefill (head dim 128 has its own kernel): the tiled kernel from 32 rows per item and KV head (where two
-    // of its waves have rows); below, four waves share the keys of 16 rows.
+    // Prefill (head dim 128 has its own kernel): the tiled kernel above 32 rows
+    // per item and KV head (where three of its waves have rows); up to there,
+    // four waves share the keys of 16 rows.
     const int64_t item_rows = g.max_query_len * group;
     const int64_t units = g.num_items * g.kv_heads;
     // 128 rows per workgroup where that leaves one for every CU (4 x 512

@@ -801,8 +801,11 @@ embed_rope_kernel(const int64_t* __restrict__ ids, const int64_t* __restrict__ p
                   U16x8* __restrict__ cos_out, U16x8* __restrict__ sin_out) {
     const int64_t t = blockIdx.x;
     const int64_t id = ids[t], pos = positions[t];
-    // An id or position outside its table reads nothing: NaN rows (the
-    // all-ones pattern), which no later step can take for an answer.
+    // An id or position outside its table reads nothing and gives a NaN row
+    // (the all-ones pattern). Nothing later refuses those: NaN keys and values
+    // go into the cache, and the sampler, to which a NaN is the largest, returns
+    // token 0. Ids and positions are for the caller to check (the runner does,
+    // on the host).
     const bool id_ok = id >= 0 && id < vocab, pos_ok = pos >= 0 && pos < max_position;
     const U16x8 bad{{~0u, ~0u, ~0u, ~0u}};
     for (int i = threadIdx.x; i < width8 + 2 * half8; i += kGatherThreads) {

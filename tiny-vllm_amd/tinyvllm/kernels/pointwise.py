@@ -253,7 +253,8 @@ def embed_rope(
     1, half] in one launch: bit copies of ``embedding[input_ids]``,
     ``cos[positions]`` and ``sin[positions]`` (tables ``[rows, columns]`` of
     one half dtype, columns a multiple of 8). Ids and positions must lie in
-    their tables; others give rows of NaNs."""
+    their tables, which the caller checks: others give rows of NaNs, and a
+    step over those samples token 0."""
     lib = load_kernels()
     device = require_gpu(input_ids, positions, embedding, cos, sin)
     for tensor in (input_ids, positions):
