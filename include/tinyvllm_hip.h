@@ -153,9 +153,10 @@ int64_t tvllm_paged_decode_split_plan(int64_t num_rows, int64_t num_heads,
  * alignment runs a workgroup of four waves per row, KV head and group of up
  * to 16 query heads, sharing each K/V load; when such units are few, each
  * row's keys split over several workgroups and a second launch merges their
- * partials. Head dims 32, 64, 128 and 256 with 16-byte aligned cache rows (8-byte ones of FP8) use
- * MFMAs there too (fp32 sums, weights as two 16-bit terms), others fp32
- * arithmetic on the vector units.
+ * partials. Head dims 32, 64, 128 and 256 with 16-byte aligned cache rows
+ * (8-byte ones of FP8) use MFMAs there too (fp32 sums; weights as two 16-bit
+ * terms, rounded to 2^-17 of themselves in bf16, to 2^-36 of the row's largest
+ * in fp16), others fp32 arithmetic on the vector units.
  * cache_dtype: dtype (caches hold q's element type; k_scale = v_scale = 1)
  * or TVLLM_FP8_E4M3 (caches hold E4M3 bytes in the paged layout;
  * K = stored * k_scale, V = stored * v_scale).
@@ -397,9 +398,9 @@ int tvllm_resolve_tokens(int64_t* tokens, const int64_t* src, const int64_t* pre
  * head_dim 128 runs the MFMA kernel (16-byte aligned Q and cache rows, cache
  * strides in whole 8-element units). Any other head_dim <= 256 runs the
  * kernels that tvllm_paged_decode has for the other shapes: 32, 64 and 256
- * with 16-byte aligned cache rows (8-byte ones of FP8) on MFMAs (workgroups of 64 or 128 (query
- * token, query head) rows of one item and KV head, or of up to 16 where an
- * item has at most 32), others in fp32 (up to 16 rows).
+ * with 16-byte aligned cache rows (8-byte ones of FP8) on MFMAs (workgroups
+ * of 64 or 128 (query token, query head) rows of one item and KV head, or of
+ * up to 16 where an item has at most 32), others in fp32 (up to 16 rows).
  * workspace, workspace_bytes: not used (null and 0 will do). A bf16 cache's V
  * is converted to fp16 for the P.V products at head_dim 128; a workgroup in
  * which a V value of 65536 or more in magnitude, an infinity or a NaN enters a

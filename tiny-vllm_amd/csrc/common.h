@@ -146,6 +146,25 @@ __device__ __forceinline__ void unpack8(const U16x8& v, float (&out)[8]) {
     }
 }
 
+// ---------------------------------------------------- matrix products --
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// c += a b over 32 of the reduction: a's row and b's column lane % 16, elements
+// 8 * (lane / 16) .. of them in the lane; c's rows 4 * (lane / 16) .. of column
+// lane % 16.
+template <typename T>
+__device__ __forceinline__ f32x4_t mfma32(const U16x8& a, const U16x8& b, f32x4_t c) {
+    typedef T t8 __attribute__((ext_vector_type(8)));
+    if constexpr (__is_same(T, __bf16)) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(t8, a),
+                                                       __builtin_bit_cast(t8, b), c, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(t8, a),
+                                                      __builtin_bit_cast(t8, b), c, 0, 0, 0);
+    }
+}
+
 // ------------------------------------------------------ fp8 KV cache --
 // Cache rows may be stored as OCP FP8 E4M3 (max 448, no infinities) with a
 // per-cache scale: stored = fp8(clamp(x * inv_scale, -448, 448)), nearest-

@@ -226,20 +226,7 @@ __global__ void __launch_bounds__(64) general_attention_kernel(GeneralAttention 
 // V = 0, as attention sinks have it, then came out wrong: its other keys 2^22
 // below the largest 0.3 % off, 2^26 below it zero).
 
-typedef __bf16 gbf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 gf16x8 __attribute__((ext_vector_type(8)));
-typedef float gf32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ __forceinline__ gf32x4 mfma32(const U16x8& a, const U16x8& b, gf32x4 c) {
-    if constexpr (std::is_same_v<T, __bf16>) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8, a),
-                                                       __builtin_bit_cast(gbf16x8, b), c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gf16x8, a),
-                                                      __builtin_bit_cast(gf16x8, b), c, 0, 0, 0);
-    }
-}
+typedef f32x4_t gf32x4;
 
 // Elements 2 * w and 2 * w + 1 of words a (first) and b: the even (or odd)
 // elements of the two side by side.

@@ -39,20 +39,7 @@
 namespace tvllm {
 namespace {
 
-typedef __bf16 lbf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 lf16x8 __attribute__((ext_vector_type(8)));
-typedef float lf32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ __forceinline__ lf32x4 mfma32(const U16x8& a, const U16x8& b, lf32x4 c) {
-    if constexpr (std::is_same_v<T, __bf16>) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lbf16x8, a),
-                                                       __builtin_bit_cast(lbf16x8, b), c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lf16x8, a),
-                                                      __builtin_bit_cast(lf16x8, b), c, 0, 0, 0);
-    }
-}
+typedef f32x4_t lf32x4;
 
 __device__ __forceinline__ U16x8 load_once(const U16x8* p) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
