@@ -420,8 +420,16 @@ struct FirstSpecial {
 // 364 -> 177 (6.1 TB/s); 256 / 8 heads of 128 907 -> 158; 33 rows of 1-4096
 // tokens, heads of 64 165 -> 47. Two tiles per chunk rather than four
 // (142 registers, three waves per SIMD): 1-7 % at head dim 64.
+// Waves per SIMD at most. Two for fp16 at head dim 64: rows of mixed lengths run
+// faster with their workgroups spread over the CUs (33 rows of 1-4096 tokens,
+// 32 / 8 heads, 41.5 us against 46.6 with the three that registers allow), short
+// ones slower (128 x 100 12.0 against 11.4).
+template <typename T, bool F8, int D>
+constexpr int kRowsWavesMax = D == 64 && !F8 && std::is_same_v<T, _Float16> ? 2 : 8;
+
 template <typename T, bool F8, int D>
 __global__ void __launch_bounds__(64 * kRowWaves)
+    __attribute__((amdgpu_waves_per_eu(1, kRowsWavesMax<T, F8, D>)))
 rows_attention_kernel(GeneralAttention a) {
     constexpr int NT = 2;                // 16-key tiles per chunk
     constexpr int CH = 16 * NT;
