@@ -166,18 +166,29 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
     return device
 
 
+_is_compiling = torch.compiler.is_compiling
+_grad_enabled = torch.is_grad_enabled
+_transforms = torch._C._functorch.peek_interpreter_stack
+_is_tracing = torch._C._is_tracing
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+
+
 def values_only(*tensors: torch.Tensor) -> bool:
     """Whether a call asks for these tensors' values and nothing else, which is
     all that a kernel behind the C interface gives: no gradient, no
     forward-mode tangent (no_grad leaves those on), no vmap or other function
     transform, no tracing or compilation, no dispatch or function mode that
     wants to see torch's ops, no tensor subclass. A module that has a torch
-    form too takes it otherwise."""
-    return not (
-        torch.compiler.is_compiling() or torch.is_grad_enabled()
-        or forward_ad._current_level >= 0
-        or torch._C._functorch.peek_interpreter_stack() is not None
-        or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
-        or (torch._C._len_torch_function_stack() > 0
-            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
-    ) and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+    form too takes it otherwise. (Asked several times a layer: about 1 us.)"""
+    if (_is_compiling() or _grad_enabled() or forward_ad._current_level >= 0
+            or _transforms() is not None or _is_tracing() or _dispatch_modes()):
+        return False
+    if _function_modes() and any(type(m) is not DeviceContext
+                                 for m in _get_current_function_mode_stack()):
+        return False
+    for tensor in tensors:
+        kind = type(tensor)
+        if kind is not torch.Tensor and kind is not torch.nn.Parameter:
+            return False
+    return True

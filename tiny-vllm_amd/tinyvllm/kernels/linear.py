@@ -9,6 +9,7 @@ from tinyvllm.kernels._extension import (
 )
 
 MAX_ROWS = 64
+HALVES = (torch.bfloat16, torch.float16)
 
 
 def fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -16,13 +17,16 @@ def fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
     rows on the GPU in 16-byte units, widths in multiples of 32, outside
     autocast and wherever more than values is asked for (autograd, forward
     mode, transforms, tracing), which only the torch ops serve."""
-    return (values_only(x, weight) and x.dim() == 2 and x.is_cuda and x.dtype == weight.dtype
-            and x.dtype in (torch.bfloat16, torch.float16) and 0 < x.shape[0] <= MAX_ROWS
-            and weight.device == x.device
-            and not torch.is_autocast_enabled("cuda")
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.is_contiguous()
-            and weight.shape[0] % 32 == 0 and weight.shape[1] % 32 == 0
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+    if not x.is_cuda or not values_only(x, weight):
+        return False
+    rows, stride = x.shape, x.stride()
+    columns, width = weight.shape
+    return (len(rows) == 2 and 0 < rows[0] <= MAX_ROWS and x.dtype in HALVES
+            and x.dtype == weight.dtype and x.get_device() == weight.get_device()
+            and stride[1] == 1 and stride[0] % 8 == 0 and weight.is_contiguous()
+            and columns % 32 == 0 and width % 32 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, *, slices: int = 0,

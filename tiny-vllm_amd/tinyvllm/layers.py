@@ -170,6 +170,13 @@ class PackedLinear(nn.Module):
             return None
         return few_rows.few_rows_linear(x, self.weight, silu=True)
 
+    def splits_decode(self, x: torch.Tensor) -> bool:
+        """Whether ``x`` is a batch that ``decode_partials`` splits."""
+        if x.dim() != 2 or not x.is_cuda or not x.is_contiguous():
+            return False
+        rows, k = x.shape
+        return (32 <= rows <= 64 and k <= 2048) or (48 <= rows <= 64 and k >= 5120)
+
     def decode_partials(self, x: torch.Tensor, splits: int = 4) -> torch.Tensor | None:
         """fp32 [splits, rows, out] partial products over ``splits`` slices of
         the reduction axis (one batched torch.bmm), or None where one GEMM
@@ -188,12 +195,9 @@ class PackedLinear(nn.Module):
         1.41 and 1.55 -> 1.60 ms; 8B at 64 rows: no change), so only the
         0.6B width at 32-64 rows (C3: 14.9k -> 15.4k tok/s) and widths of
         5120 and more at 48-64 rows take the split."""
-        rows, k = x.shape if x.dim() == 2 else (0, 0)
-        if (not x.is_cuda or x.dim() != 2 or not x.is_contiguous() or rows > 64
-                or k % (8 * splits)):
+        if not self.splits_decode(x) or x.shape[1] % (8 * splits):
             return None
-        if not ((k <= 2048 and rows >= 32) or (k >= 5120 and rows >= 48)):
-            return None
+        rows, k = x.shape
         xs = x.view(rows, splits, k // splits).transpose(0, 1)
         ws = self.weight.view(self.weight.shape[0], splits, k // splits).permute(1, 2, 0)
         return torch.bmm(xs, ws, out_dtype=torch.float32)

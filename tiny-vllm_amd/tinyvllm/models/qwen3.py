@@ -159,6 +159,7 @@ class Qwen3Attention(nn.Module):
         # split-K partials: the fused decode kernel sums them itself.
         from_partials = getattr(attention, "attend_qkv_partials", None)
         if (from_partials is not None and attention.takes_qkv_partials(self.num_heads)
+                and self.qkv_proj.splits_decode(hidden_states)
                 and not self.qkv_proj.takes_few_rows(hidden_states)):
             parts = self.qkv_proj.decode_partials(hidden_states)
             if parts is not None:
