@@ -416,10 +416,11 @@ struct FirstSpecial {
 // Bound by the rate of its loads at many rows, by their latency along the
 // longest row at few. In us, against fp32 arithmetic on the vector units
 // (K and V broadcast to the query rows' lanes): 64 rows x 2048 tokens, 32
-// query and 8 KV heads of 64 167 -> 57 (4.7 TB/s of 128-byte pieces), of 256
-// 364 -> 177 (6.1 TB/s); 256 / 8 heads of 128 907 -> 158; 33 rows of 1-4096
-// tokens, heads of 64 165 -> 47. Two tiles per chunk rather than four
-// (142 registers, three waves per SIMD): 1-7 % at head dim 64.
+// query and 8 KV heads of 64 165 -> 46 (268 MB in graph replay, some of them
+// left in the 256 MB memory-side cache), of 256 362 -> 177 (6.1 TB/s); 256 / 8
+// heads of 128 888 -> 159; 33 rows of 1-4096 tokens, heads of 64 170 -> 52 with
+// the merge. Two tiles per chunk rather than four (148 registers at head dim
+// 64, three waves per SIMD): 1-7 % there.
 // Waves per SIMD at most. Two for fp16 at head dim 64: rows of mixed lengths run
 // faster with their workgroups spread over the CUs (33 rows of 1-4096 tokens,
 // 32 / 8 heads, 41.5 us against 46.6 with the three that registers allow), short
@@ -797,9 +798,9 @@ rows_attention_kernel(GeneralAttention a) {
 // against 48 MFMAs per 32 keys at head dim 256) and by LDS bandwidth at RT = 1
 // (1 KiB of operand per 16-cycle MFMA and wave). Registers are held to 256, so
 // that two waves share a SIMD. In us, against the vector-unit kernel: 4 x 512
-// queries over 2048 tokens, 32 query and 8 KV heads of 64 2257 -> 84 (357
-// TFLOP/s), of 256 6566 -> 329 (366 TFLOP/s); 2 x 256 over 1033, 16 / 8 heads
-// of 256 488 -> 53.
+// queries over 2048 tokens, 32 query and 8 KV heads of 64 2241 -> 81 (370
+// TFLOP/s), of 256 6520 -> 303 (397 TFLOP/s); 2 x 256 over 1033, 16 / 8 heads
+// of 256 482 -> 50.
 template <typename T, bool F8, int D, int RT, int HV>
 __global__ void __launch_bounds__(64 * kRowWaves * HV, 2)
 tiles_attention_kernel(GeneralAttention a) {
@@ -1294,9 +1295,10 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
     const int64_t item_rows = g.max_query_len * group;
     const int64_t units = g.num_items * g.kv_heads;
     // 128 rows per workgroup where that leaves one for every CU (4 x 512
-    // queries over 2048 tokens, 32 / 8 heads of 64: 84 us against 99 with 64
-    // rows; heads of 256 gain nothing, 320 against 329, and lose where tiles
-    // are few, 72 against 63 us for 3 x 300).
+    // queries over 2048 tokens, 32 / 8 heads of 64: 81 us against 94 with 64
+    // rows; where tiles are few they lose, 41 against 38 us for 3 x 300 over
+    // 1300, 62 against 34 for 8 x 40 over 2040). Heads of 256 have no registers
+    // for a second row tile.
     const bool wide = D <= 64 && units * ((item_rows + 127) / 128) >= 256;
     const int64_t ty = (item_rows + (wide ? 127 : 63)) / (wide ? 128 : 64);
     const bool tiles = rows_kernel && D != 128 && !g.rows && item_rows > 2 * GH && ty <= 65535;
@@ -1326,9 +1328,10 @@ int launch_general_attention(const GeneralAttention& g_in, hipStream_t stream) {
         using T = typename Elem<DT>::T;
         if (tiles) {
             // Where the tiles do not fill the CUs, two halves of a workgroup
-            // share the keys (2 x 256 over 1033, heads of 256: 61 -> 53 us; 8
-            // x 40 over 2040, FP8, heads of 64: 43 -> 35 us); at full grids
-            // the halves only add their merge (99 -> 112 us).
+            // share the keys (2 x 256 over 1033, heads of 256: 59 -> 50 us; 8
+            // x 40 over 2040, FP8, heads of 64: 42 -> 34 us); at full grids
+            // the halves only add their merge (4 x 512 over 2048 in tiles of
+            // 64 rows, heads of 64 / 256: 94 -> 109, 303 -> 318 us).
             const bool halves = units * ty < 256;
             const dim3 tg{static_cast<uint32_t>(units), static_cast<uint32_t>(ty), 1u};
             auto go = [&]<int DD, int RT, int HV>() {

@@ -540,12 +540,13 @@ sample_kernel(const T* __restrict__ logits, int64_t vocab, int64_t stride,
 // elements each, one 256-thread workgroup): three launches of rows x spans
 // workgroups that each read the row once, and a short one per row, where the
 // one-workgroup kernel reads the row about fifteen times from one CU. 64 rows
-// x 151936 bf16 with mixed filters: 1965 -> 68 us (race about 30, bins 17,
-// finish 10-16, maxima 10: four dependent launches of one or two waves per SIMD;
+// x 151936 bf16 with mixed filters: 1965 -> 71 us (in a trace race 26, finish
+// 17, bins 16, maxima 9: four dependent launches of one or two waves per SIMD;
 // 19 MB is 3 us of memory. Two changes left the race where it is: ruling
-// tokens out by a bound of one exponential before the two logarithms, 71, and
-// a rolled loop of a quarter of its 58 KB of instructions, 69). A batch of greedy
-// rows pays 2 us for the two launches that find nothing to do.
+// tokens out by a bound of one exponential before the two logarithms and a
+// rolled loop of a quarter of its 58 KB of instructions). A batch of greedy
+// rows pays 0.6 us (bf16) to 1.5 us (fp32) for the two launches that find
+// nothing to do.
 //
 //   argmax_part_kernel  each span's maximum; clears the row's bins.
 //   bins_kernel         the row maximum from the spans (greedy rows are done);
